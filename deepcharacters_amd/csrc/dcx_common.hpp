@@ -42,4 +42,24 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Smallest value of a group of 4, 16 or 64 lanes (all of them active), valid in
+// every lane: DPP row operations, which need no LDS crossbar round trip, and
+// for the whole wavefront the four rows' results through scalar registers.
+template <int kLanes>
+__device__ __forceinline__ unsigned group_min(unsigned v) {
+  static_assert(kLanes == 4 || kLanes == 16 || kLanes == 64, "a quad, a DPP row or a wavefront");
+  v = min(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false));  // [1,0,3,2]
+  v = min(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xf, 0xf, false));  // [2,3,0,1]
+  if (kLanes >= 16) {
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x141, 0xf, 0xf, false));  // half mirror
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x140, 0xf, 0xf, false));  // mirror
+  }
+  if (kLanes == 64) {
+    const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 15), b = (unsigned)__builtin_amdgcn_readlane((int)v, 31);
+    const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)v, 47), d = (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+    v = min(min(a, b), min(c, d));
+  }
+  return v;
+}
+
 }  // namespace dcx

@@ -64,3 +64,39 @@ def test_dt_loss_forward_backward_match_oracle():
     tp = _t(pts).requires_grad_(True)
     (dtloss.DTLossFn.apply(tp, _t(isb, torch.uint8), dist, _t(crops)) * _t(g)).sum().backward()
     np.testing.assert_allclose(tp.grad.cpu().numpy(), gp, rtol=1e-6, atol=1e-6)
+
+
+def _shapes(kind, rng, V, H, W):
+    if kind == "sparse":
+        return rng.uniform(size=(V, H, W)) < 3.0 / (H * W)
+    if kind == "dense":
+        return rng.uniform(size=(V, H, W)) < 0.7
+    if kind == "ends":  # the nearest column jumps from one side to the other
+        m = np.zeros((V, H, W), bool)
+        m[:, :, :1] = m[:, :, -1:] = True
+        return m
+    return np.broadcast_to(np.array([False, True])[np.arange(V) % 2][:, None, None], (V, H, W)).copy()  # empty, full
+
+
+@pytest.mark.parametrize("kind", ["sparse", "dense", "ends", "plain"])
+@pytest.mark.parametrize("H,W", [(1, 70), (2, 1), (2, 3), (31, 4), (32, 5), (33, 63), (64, 64), (65, 255), (3, 256),
+                                 (40, 257), (97, 1025), (5, 4096), (4096, 6), (3, 4097), (4097, 3)])
+def test_transforms_at_the_edges_of_words_rows_and_sizes(kind, H, W):
+    """Whole squared distances and encoded bytes, so no tolerance: dist is the
+    rounded root of a whole number below 2^25."""
+    m = _shapes(kind, np.random.default_rng(H * 7 + W), 3, H, W)
+    dist = dtloss.edt(_t(m, torch.uint8)).cpu().numpy()
+    enc = dtloss.dt_encode(_t(m, torch.uint8)).cpu().numpy()
+    for v in range(len(m)):
+        if not m[v].any():
+            assert np.all(np.isinf(dist[v])) and np.all(enc[v] == 255)
+            continue
+        out = ndimage.distance_transform_edt(~m[v])
+        assert np.array_equal(dist[v], np.sqrt(np.rint(out ** 2).astype(np.float32)))
+        # without any background the inside distance is the farthest value
+        inside = ndimage.distance_transform_edt(m[v]) if not m[v].all() else np.full((H, W), 1e30)
+        ref = np.where(m[v], np.clip(np.rint(inside) - 1, 0, 126), 127 + np.clip(np.rint(out / 2), 1, 128))
+        pad = np.pad(m[v], 1)
+        near = [pad[:-2, 1:-1], pad[2:, 1:-1], pad[1:-1, :-2], pad[1:-1, 2:]]
+        ref[np.any([n != m[v] for n in near], axis=0)] = 127
+        assert np.array_equal(enc[v], ref.astype(np.uint8))
