@@ -5,17 +5,16 @@
 // The data->model term searches, for each DT boundary pixel, the nearest
 // boundary point within 30*scale.  DCX_SIL_BRUTE scans every point as the
 // reference does (MultiViewSilhouetteLossGPUOp.cu:195-212).  DCX_SIL_BINNED
-// first buckets the view's boundary points into a uniform grid whose cells
-// are slightly larger than the search radius, then scans only the 3x3 cells
-// around the pixel; it evaluates the same float distance and keeps the
-// lexicographic minimum of (distance, index), so both paths return the same
-// ids as the reference's strict-< scan (lowest index among equal distances).
+// first buckets the view's boundary points into a uniform grid of cells an
+// eighth of the search radius wide.  A wavefront takes a boundary pixel and
+// scans the 3x3 cells around it, then, only if something beyond them could
+// still be nearer, all cells within the best distance so far; it evaluates
+// the same float distance and keeps the lexicographic minimum of (distance,
+// index), so both paths return the same ids as the reference's strict-< scan
+// (lowest index among equal distances).
 #include "raster_internal.hpp"
 
 namespace dcx {
-
-dcx_status exclusive_scan(const unsigned int* in, unsigned int* out, unsigned int* aux, long long n,
-                          hipStream_t s);
 
 namespace {
 
@@ -36,21 +35,50 @@ struct SilArgs {
   float* cid;            // [B,C,U,V]
 };
 
+constexpr int kCellsPerRadius = 8;
+constexpr int kListStride = 32;  // a counter per 128-byte line
+
 struct GridArgs {
   int gx, gy, cells_per_view;
-  unsigned int* cnt;     // [views*cells]
-  unsigned int* off;     // [views*cells + 1]
-  unsigned int* fill;
-  unsigned int* items;   // point ids, capacity = B*C*N
+  unsigned int* cnt;     // [views, cells]; null: no grid (brute force)
+  unsigned int* off;     // [views, cells + 1], from each view's first item
+  f4* items;             // [views, N] (u, v, point id) by cell
+  unsigned int* list_n;  // [views, kListStride] boundary pixels found so far
+  unsigned int* list;    // [views, U * V] their indices in the view
 };
 
+struct GridGeom {
+  float ox, oy, cell;
+};
+
+__device__ __forceinline__ GridGeom grid_geom(const float* cr) {
+  const float sc = cr[2];
+  const float R = 30.f * sc * (1.f + 1.f / 1024.f);
+  GridGeom g;
+  g.cell = R / (float)kCellsPerRadius;
+  g.ox = (0.f - cr[0]) * sc + cr[3] - 2.f * R;
+  g.oy = (0.f - cr[1]) * sc + cr[4] - 2.f * R;
+  return g;
+}
+
+__device__ __forceinline__ int cell_of(const GridGeom& g, const GridArgs& ga, float x, float y) {
+  const float fx = floorf((x - g.ox) / g.cell), fy = floorf((y - g.oy) / g.cell);
+  if (!(fx >= 0.f && fy >= 0.f && fx < (float)ga.gx && fy < (float)ga.gy)) return -1;
+  return (int)fy * ga.gx + (int)fx;
+}
+
 // Model->data residual per (batch, camera, point): MultiViewSilhouetteLossGPUOp.cu:11-138.
-__global__ __launch_bounds__(kB) void sil_point_kernel(SilArgs a) {
+// Boundary points are also counted into their grid cells.
+__global__ __launch_bounds__(kB) void sil_point_kernel(SilArgs a, GridArgs g) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
   if (i >= (long long)a.B * a.C * a.N) return;
   const int view = (int)(i / a.N);
   const float* cr = a.crops + (size_t)view * 7;
   const float pu = a.pts[2 * i], pv = a.pts[2 * i + 1];
+  if (g.cnt && a.isb[i]) {
+    const int c = cell_of(grid_geom(cr), g, pu, pv);
+    if (c >= 0) atomicAdd(g.cnt + (size_t)view * g.cells_per_view + c, 1u);
+  }
   const bool in_view = pu - 2 > cr[3] && pu + 2 < cr[5] && pv - 2 > cr[4] && pv + 2 < cr[6];
   const float fx = (pu - cr[3]) / cr[2] + cr[0], fy = (pv - cr[4]) / cr[2] + cr[1];
   const int x = (int)fx, y = (int)fy;
@@ -83,14 +111,22 @@ __global__ __launch_bounds__(kB) void sil_point_kernel(SilArgs a) {
   a.res[i] = dv * (1.f / (255.f));
 }
 
+// Value 127 and at least four 127s in the 5x5 window (pixels outside the image
+// not counted).  The window's loads are issued together, clamped to the image.
 __device__ __forceinline__ bool is_dt_boundary(const unsigned char* img, int U, int V, int ui, int vi) {
   if (img[(size_t)vi * U + ui] != 127) return false;
   int counter = 0;
-  for (int j = -2; j <= 2; ++j)
+#pragma unroll
+  for (int j = -2; j <= 2; ++j) {
+    const int yy = vi + j;
+    const unsigned char* row = img + (size_t)min(max(yy, 0), V - 1) * U;
+#pragma unroll
     for (int i = -2; i <= 2; ++i) {
-      const int yy = vi + j, xx = ui + i;
-      if (yy >= 0 && yy < V && xx >= 0 && xx < U && img[(size_t)yy * U + xx] == 127) counter++;
+      const int xx = ui + i;
+      const bool in = yy >= 0 && yy < V && xx >= 0 && xx < U;
+      counter += (row[min(max(xx, 0), U - 1)] == 127) & in;
     }
+  }
   return counter >= 4;
 }
 
@@ -135,78 +171,149 @@ __global__ __launch_bounds__(kB) void sil_pixel_brute_kernel(SilArgs a) {
   write_d2m(a, o, view, best, ix, iy, sc);
 }
 
-struct GridGeom {
-  float ox, oy, cell;
-};
-
-__device__ __forceinline__ GridGeom grid_geom(const float* cr) {
-  const float sc = cr[2];
-  const float R = 30.f * sc;
-  GridGeom g;
-  g.cell = R * (1.f + 1.f / 1024.f);
-  g.ox = (0.f - cr[0]) * sc + cr[3] - 2.f * g.cell;
-  g.oy = (0.f - cr[1]) * sc + cr[4] - 2.f * g.cell;
-  return g;
-}
-
-__device__ __forceinline__ int cell_of(const GridGeom& g, const GridArgs& ga, float x, float y) {
-  const float fx = floorf((x - g.ox) / g.cell), fy = floorf((y - g.oy) / g.cell);
-  if (!(fx >= 0.f && fy >= 0.f && fx < (float)ga.gx && fy < (float)ga.gy)) return -1;
-  return (int)fy * ga.gx + (int)fx;
-}
-
-__global__ __launch_bounds__(kB) void sil_grid_count_kernel(SilArgs a, GridArgs g) {
+__global__ __launch_bounds__(kB) void clear_u32_kernel(unsigned int* __restrict__ p, long long n) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)a.B * a.C * a.N || !a.isb[i]) return;
-  const int view = (int)(i / a.N);
-  const GridGeom gg = grid_geom(a.crops + (size_t)view * 7);
-  const int c = cell_of(gg, g, a.pts[2 * i], a.pts[2 * i + 1]);
-  if (c >= 0) atomicAdd(g.cnt + (size_t)view * g.cells_per_view + c, 1u);
+  if (i < n) p[i] = 0u;
 }
 
+// Cell offsets of one view per workgroup: every view has its own N item slots,
+// so no scan crosses views.
+__global__ __launch_bounds__(1024) void sil_grid_scan_kernel(GridArgs g) {
+  __shared__ unsigned int s_wave[16];
+  const unsigned int* cnt = g.cnt + (size_t)blockIdx.x * g.cells_per_view;
+  unsigned int* off = g.off + (size_t)blockIdx.x * (g.cells_per_view + 1);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  unsigned int base = 0;
+  for (int c0 = 0; c0 < g.cells_per_view; c0 += 4096) {
+    const int c = c0 + 4 * (int)threadIdx.x;
+    unsigned int v[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { v[k] = c + k < g.cells_per_view ? cnt[c + k] : 0u; sum += v[k]; }
+    unsigned int inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned int o = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += o;
+    }
+    if (lane == 63) s_wave[wid] = inc;
+    __syncthreads();
+    unsigned int before = base, total = 0;
+    for (int w = 0; w < 16; ++w) {
+      before += w < wid ? s_wave[w] : 0u;
+      total += s_wave[w];
+    }
+    before += inc - sum;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (c + k < g.cells_per_view) off[c + k] = before;
+      before += v[k];
+    }
+    base += total;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) off[g.cells_per_view] = base;
+}
+
+// The boundary points into their cells' slots, last slot first (the counts are
+// used up; the order in a cell changes no result).
 __global__ __launch_bounds__(kB) void sil_grid_scatter_kernel(SilArgs a, GridArgs g) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
   if (i >= (long long)a.B * a.C * a.N || !a.isb[i]) return;
   const int view = (int)(i / a.N);
-  const GridGeom gg = grid_geom(a.crops + (size_t)view * 7);
-  const int c = cell_of(gg, g, a.pts[2 * i], a.pts[2 * i + 1]);
+  const float x = a.pts[2 * i], y = a.pts[2 * i + 1];
+  const int c = cell_of(grid_geom(a.crops + (size_t)view * 7), g, x, y);
   if (c < 0) return;
-  const size_t cell = (size_t)view * g.cells_per_view + c;
-  g.items[g.off[cell] + atomicAdd(g.fill + cell, 1u)] = (unsigned int)(i - (long long)view * a.N);
+  const unsigned int slot = g.off[(size_t)view * (g.cells_per_view + 1) + c] +
+                            atomicSub(g.cnt + (size_t)view * g.cells_per_view + c, 1u) - 1u;
+  g.items[(size_t)view * a.N + slot] = mk4(x, y, __int_as_float((int)(i - (long long)view * a.N)), 0.f);
 }
 
-__global__ __launch_bounds__(kB) void sil_pixel_binned_kernel(SilArgs a, GridArgs g) {
-  const long long o = (long long)blockIdx.x * kB + threadIdx.x;
-  const long long UV = (long long)a.U * a.V;
-  if (o >= (long long)a.B * a.C * UV) return;
-  const int view = (int)(o / UV);
-  const int p = (int)(o - (long long)view * UV);
-  const int ui = p % a.U, vi = p / a.U;
-  const unsigned char* img = a.dt + (size_t)view * UV;
-  int best = -1;
-  float ix = 0.f, iy = 0.f, sc = 1.f;
-  if (is_dt_boundary(img, a.U, a.V, ui, vi)) {
+// Nearest of the points in the cells within `ring` of (cx, cy), by a whole
+// wavefront: four cell rows at a time, 16 lanes a row (a row's cells are one
+// range of items).  Each lane updates its own (bd, best).
+__device__ __forceinline__ void scan_ring(const GridArgs& g, const unsigned int* off, const f4* items, int cx, int cy,
+                                          int ring, float ix, float iy, float& bd, int& best) {
+  const int lane = threadIdx.x & 63;
+  const int x0 = max(cx - ring, 0), x1 = min(cx + ring, g.gx - 1);
+  const int y1 = min(cy + ring, g.gy - 1);
+  if (x0 > x1) return;
+  for (int yy = max(cy - ring, 0) + (lane >> 4); yy <= y1; yy += 4) {
+    const unsigned int end = off[yy * g.gx + x1 + 1];
+    // two items in flight; past the end the last one again, which changes nothing
+    for (unsigned int k = off[yy * g.gx + x0] + (lane & 15); k < end; k += 32) {
+      const f4 it[2] = {items[k], items[min(k + 16, end - 1)]};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float dx = it[j].x - ix, dy = it[j].y - iy;
+        const float d = sqrtf(dx * dx + dy * dy);
+        const int v = __float_as_int(it[j].z);
+        if (d < bd || (d == bd && best >= 0 && v < best)) { bd = d; best = v; }
+      }
+    }
+  }
+}
+
+// Smallest (distance, index) over the wavefront, the result in every lane.
+__device__ __forceinline__ void nearest_of_wave(float& bd, int& best) {
+  const unsigned d = best >= 0 ? __float_as_uint(bd) : 0xffffffffu;  // distances are not negative: bit order
+  const unsigned m = group_min<64>(d);
+  best = (int)group_min<64>(d == m ? (unsigned)best : 0xffffffffu);
+  if (m != 0xffffffffu) bd = __uint_as_float(m);
+}
+
+// The boundary pixels' indices into their view's list, one reservation per
+// workgroup; every other pixel gets its empty result.
+__global__ __launch_bounds__(kB) void sil_pixel_list_kernel(SilArgs a, GridArgs g) {
+  __shared__ unsigned int s_n, s_at;
+  const int view = blockIdx.y, UV = a.U * a.V, p = blockIdx.x * kB + threadIdx.x;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  unsigned int mine = 0;
+  bool found = false;
+  if (p < UV) {
+    found = is_dt_boundary(a.dt + (size_t)view * UV, a.U, a.V, p % a.U, p / a.U);
+    if (found) mine = atomicAdd(&s_n, 1u);
+    else write_d2m(a, (size_t)view * UV + p, view, -1, 0.f, 0.f, 1.f);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_n) s_at = atomicAdd(g.list_n + view * kListStride, s_n);
+  __syncthreads();
+  if (found) g.list[(size_t)view * UV + s_at + mine] = (unsigned int)p;
+}
+
+// A wavefront per listed pixel.  (Contour pixels cluster: dealt out by the
+// workgroup that finds them, a few workgroups searched for a whole horizontal
+// edge while the rest of the chip was done.)  16 views of 256 x 256 with 50k
+// points each, an eighth of them on the boundary: 3.49 ms with a lane per
+// pixel over cells as wide as the radius, 0.06 with the list; what is left is
+// the chain list -> cell offsets -> points of each search.
+constexpr int kSearchBlocks = 256;  // per view
+__global__ __launch_bounds__(kB) void sil_search_kernel(SilArgs a, GridArgs g) {
+  const int view = blockIdx.y, UV = a.U * a.V;
+  const unsigned int n = g.list_n[view * kListStride];
+  for (unsigned int q = (blockIdx.x * kB + threadIdx.x) >> 6; q < n; q += kSearchBlocks * (kB / 64)) {
+    const int p = __builtin_amdgcn_readfirstlane((int)g.list[(size_t)view * UV + q]);
+    const int ui = p % a.U, vi = p / a.U;
     const float* cr = a.crops + (size_t)view * 7;
-    sc = cr[2];
-    ix = ((float)ui - cr[0]) * sc + cr[3];
-    iy = ((float)vi - cr[1]) * sc + cr[4];
-    const float R = 30.f * sc;
-    float bd = R;
+    const float sc = cr[2];
+    const float ix = ((float)ui - cr[0]) * sc + cr[3], iy = ((float)vi - cr[1]) * sc + cr[4];
     const GridGeom gg = grid_geom(cr);
     const int cx = (int)floorf((ix - gg.ox) / gg.cell), cy = (int)floorf((iy - gg.oy) / gg.cell);
-    const float* pv = a.pts + (size_t)view * a.N * 2;
-    for (int yy = max(cy - 1, 0); yy <= min(cy + 1, g.gy - 1); ++yy)
-      for (int xx = max(cx - 1, 0); xx <= min(cx + 1, g.gx - 1); ++xx) {
-        const size_t cell = (size_t)view * g.cells_per_view + yy * g.gx + xx;
-        for (unsigned int k = g.off[cell]; k < g.off[cell + 1]; ++k) {
-          const int v = (int)g.items[k];
-          const float dx = pv[2 * v] - ix, dy = pv[2 * v + 1] - iy;
-          const float d = sqrtf(dx * dx + dy * dy);
-          if (d < bd || (d == bd && best >= 0 && v < best)) { bd = d; best = v; }
-        }
-      }
+    const unsigned int* off = g.off + (size_t)view * (g.cells_per_view + 1);
+    const f4* items = g.items + (size_t)view * a.N;
+    float bd = 30.f * sc;
+    int best = -1;
+    scan_ring(g, off, items, cx, cy, 1, ix, iy, bd, best);
+    nearest_of_wave(bd, best);
+    // a point outside the cells within r of the pixel's is farther than
+    // r * step (the margin covers the rounding of positions to cells)
+    const float step = gg.cell * (1.f - 1.f / 256.f);
+    if (!(bd < step)) {
+      scan_ring(g, off, items, cx, cy, min((int)(bd / step) + 1, kCellsPerRadius + 1), ix, iy, bd, best);
+      nearest_of_wave(bd, best);
+    }
+    if ((threadIdx.x & 63) == 0) write_d2m(a, (size_t)view * UV + p, view, best, ix, iy, sc);
   }
-  write_d2m(a, o, view, best, ix, iy, sc);
 }
 
 __global__ __launch_bounds__(kB) void sil_bwd_point_kernel(const float* __restrict__ g, const float* __restrict__ dtg,
@@ -333,18 +440,36 @@ __global__ __launch_bounds__(kB) void cov_project_kernel(const float* __restrict
   uv[2 * i + 1] = p.y;
 }
 
-__device__ __forceinline__ f3 uv2bary(float u, float v, f2 a, f2 b, f2 c) {
-  const float e2 = ((a.y - b.y) * u + (b.x - a.x) * v + a.x * b.y - b.x * a.y) /
-                   ((a.y - b.y) * c.x + (b.x - a.x) * c.y + a.x * b.y - b.x * a.y);
-  const float e1 = ((a.y - c.y) * u + (c.x - a.x) * v + a.x * c.y - c.x * a.y) /
-                   ((a.y - c.y) * b.x + (c.x - a.x) * b.y + a.x * c.y - c.x * a.y);
-  return mk3(1.f - e2 - e1, e1, e2);
-}
+// uv2barycentric's weights of corners b and c are quotients num / den whose
+// denominators are the triangle's; the first weight is 1 minus both.
+struct EdgeQuotient {
+  float dy, dx, pq, qp, den, r;
+  // the line through p and q, with weight 1 at o; r is 1 / den to a few ulp
+  __device__ __forceinline__ EdgeQuotient(f2 p, f2 q, f2 o)
+      : dy(p.y - q.y), dx(q.x - p.x), pq(p.x * q.y), qp(q.x * p.y) {
+    den = num(o.x, dx * o.y);
+    r = __builtin_amdgcn_rcpf(den);
+  }
+  __device__ __forceinline__ float num(float u, float dxv) const { return dy * u + dxv + pq - qp; }
+  // far from the ends of the exponent range: no overflow, no flushed reciprocal
+  __device__ __forceinline__ bool plain() const {
+    return fabsf(den) > 1e-30f && fabsf(den) < 1e30f && fabsf(pq) < 1e30f && fabsf(qp) < 1e30f;
+  }
+};
 
+// Eight lanes per (view, face), one row of its pixel box each.  A weight is
+// compared with the limits as a product with the reciprocal, within 1e-6 of
+// the quotient where it is near them, so the two divisions are made only for
+// pixels within 1e-5 of a limit, and for triangles near the ends of the
+// exponent range.  A lane per face walked boxes of 34 x 34 pixels (the long
+// triangles of a cap, 64 of them in one wavefront) after the rest of the
+// launch was done.  16 views of 1285 x 940, 100k faces: 294 -> 107 us, which is
+// the issue time of its vector instructions.
+constexpr int kCovLanes = 8;
 __global__ __launch_bounds__(kB) void cov_raster_kernel(const float* __restrict__ uv, const int* __restrict__ faces,
                                                          int B, int C, int N, int F, int H, int W,
                                                          unsigned char* __restrict__ cov) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
+  const long long i = ((long long)blockIdx.x * kB + threadIdx.x) / kCovLanes;
   if (i >= (long long)B * C * F) return;
   const int view = (int)(i / F), f = (int)(i - (long long)view * F);
   const f2* P = (const f2*)uv + (size_t)view * N;
@@ -353,13 +478,27 @@ __global__ __launch_bounds__(kB) void cov_raster_kernel(const float* __restrict_
   const float by0 = fmaxf(fminf(p0.y, fminf(p1.y, p2.y)) - 0.5f, 0.f);
   const float bx1 = fminf(fmaxf(p0.x, fmaxf(p1.x, p2.x)) + 0.5f, (float)(W - 1));
   const float by1 = fminf(fmaxf(p0.y, fmaxf(p1.y, p2.y)) + 0.5f, (float)(H - 1));
-  unsigned char* cv = cov + (size_t)view * H * W;
-  for (int u = (int)bx0; (float)u <= bx1; ++u)
-    for (int v = (int)by0; (float)v <= by1; ++v) {
-      const f3 e = uv2bary((float)u + 0.5f, (float)v + 0.5f, p0, p1, p2);
-      if (e.x >= -0.001f && e.y >= -0.001f && e.z >= -0.001f && e.x <= 1.001f && e.y <= 1.001f && e.z <= 1.001f)
-        cv[(size_t)v * W + u] = 1;
+  // first weights 1 at p1 and p2; e0 = 1 - e2 - e1
+  const EdgeQuotient q1(p0, p2, p1), q2(p0, p1, p2);
+  const bool plain = q1.plain() && q2.plain();
+  constexpr float kLo = -0.001f, kHi = 1.001f, kMargin = 1e-5f;
+  const int ue = bx1 >= 0.f ? (int)bx1 : -1, ve = by1 >= 0.f ? (int)by1 : -1;  // the last u, v with (float)u <= bx1
+  for (int v = (int)by0 + (int)(threadIdx.x % kCovLanes); v <= ve; v += kCovLanes) {
+    unsigned char* row = cov + (size_t)view * H * W + (size_t)v * W;
+    const float py = (float)v + 0.5f, r1 = q1.dx * py, r2 = q2.dx * py;
+    for (int u = (int)bx0; u <= ue; ++u) {
+      const float n1 = q1.num((float)u + 0.5f, r1), n2 = q2.num((float)u + 0.5f, r2);
+      const float a1 = n1 * q1.r, a2 = n2 * q2.r, a0 = 1.f - a2 - a1;
+      const float lo = fminf(a0, fminf(a1, a2)), hi = fmaxf(a0, fmaxf(a1, a2));
+      if (plain && (lo < kLo - kMargin || hi > kHi + kMargin)) continue;
+      bool in = true;
+      if (!(plain && lo > kLo + kMargin && hi < kHi - kMargin)) {
+        const float e2 = n2 / q2.den, e1 = n1 / q1.den, e0 = 1.f - e2 - e1;
+        in = e0 >= kLo && e1 >= kLo && e2 >= kLo && e0 <= kHi && e1 <= kHi && e2 <= kHi;
+      }
+      if (in) row[u] = 1;
     }
+  }
 }
 
 // The boundary test of boundary_kernel on the coverage bitmap (1 = covered).
@@ -381,29 +520,34 @@ __global__ __launch_bounds__(kB) void cov_boundary_kernel(const unsigned char* _
   out[i] = f;
 }
 
+// 16 bytes a lane where the array starts on 16 bytes, the rest byte by byte.
 __global__ __launch_bounds__(kB) void fill_u8_kernel(unsigned char* __restrict__ p, long long n) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i < n) p[i] = 0;
+  const long long i = 16 * ((long long)blockIdx.x * kB + threadIdx.x);
+  if (((uintptr_t)p & 15) == 0 && i + 16 <= n) {
+    *reinterpret_cast<uint4*>(p + i) = make_uint4(0u, 0u, 0u, 0u);
+  } else {
+    for (int k = 0; k < 16 && i + k < n; ++k) p[i + k] = 0;
+  }
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct SilWs {
   int gx, gy;
-  size_t cnt, off, fill, aux, items, total;
+  size_t cnt, off, items, list, total;
 };
 
+// The grid reaches 2 radii beyond the DT image on every side.
 SilWs sil_ws(int B, int C, int N, int U, int V) {
   SilWs w{};
-  w.gx = U / 30 + 6;
-  w.gy = V / 30 + 6;
-  const size_t cells = (size_t)B * C * w.gx * w.gy;
+  w.gx = kCellsPerRadius * (U / 30 + 6);
+  w.gy = kCellsPerRadius * (V / 30 + 6);
+  const size_t views = (size_t)B * C, cells = (size_t)w.gx * w.gy;
   size_t o = 0;
-  w.cnt = o; o = align256(o + 4 * cells);
-  w.off = o; o = align256(o + 4 * (cells + 1));
-  w.fill = o; o = align256(o + 4 * cells);
-  w.aux = o; o = align256(o + 4 * ((cells + 1023) / 1024 + 1));
-  w.items = o; o = align256(o + 4 * (size_t)B * C * N);
+  w.cnt = o; o = align256(o + 4 * views * (cells + kListStride));  // the lists' lengths behind the counts
+  w.off = o; o = align256(o + 4 * views * (cells + 1));
+  w.items = o; o = align256(o + sizeof(f4) * views * N);
+  w.list = o; o = align256(o + 4 * views * U * V);
   w.total = o;
   return w;
 }
@@ -431,24 +575,28 @@ extern "C" dcx_status dcx_mvsil_fwd(const float* points, const float* normals, c
   SilArgs a{B, C, N, U, V, points, normals, is_boundary, dt_image, crops, residual, residual1, dt_image_gradient,
             closest_vertex_id};
   const long long P = (long long)B * C * N, PIX = (long long)B * C * U * V;
-  hipLaunchKernelGGL(sil_point_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a);
   if (search == DCX_SIL_BRUTE) {
+    hipLaunchKernelGGL(sil_point_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, GridArgs{});
     hipLaunchKernelGGL(sil_pixel_brute_kernel, dim3(ceil_div(PIX, kB)), dim3(kB), 0, s, a);
     return check_launch("dcx_mvsil_fwd(brute)");
   }
   const SilWs L = sil_ws(B, C, N, U, V);
   DCX_REQUIRE(workspace && ws_bytes >= L.total, "dcx_mvsil_fwd: workspace %zu < %zu", ws_bytes, L.total);
+  const long long radii = (long long)B * C * (U / 30 + 6) * (V / 30 + 6);
+  DCX_REQUIRE(radii <= 4096ll * 1024, "dcx_mvsil_fwd: a grid of %lld search radii exceeds 4M", radii);
   char* w = (char*)workspace;
-  GridArgs g{L.gx, L.gy, L.gx * L.gy, (unsigned int*)(w + L.cnt), (unsigned int*)(w + L.off),
-             (unsigned int*)(w + L.fill), (unsigned int*)(w + L.items)};
+  GridArgs g{L.gx, L.gy, L.gx * L.gy, (unsigned int*)(w + L.cnt), (unsigned int*)(w + L.off), (f4*)(w + L.items),
+             nullptr, (unsigned int*)(w + L.list)};
   const long long cells = (long long)B * C * g.cells_per_view;
-  DCX_HIP(hipMemsetAsync(g.cnt, 0, 4 * cells, s));
-  DCX_HIP(hipMemsetAsync(g.fill, 0, 4 * cells, s));
-  hipLaunchKernelGGL(sil_grid_count_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, g);
-  dcx_status st = exclusive_scan(g.cnt, g.off, (unsigned int*)(w + L.aux), cells, s);
-  if (st) return st;
+  g.list_n = g.cnt + cells;
+  const long long clear = cells + (long long)B * C * kListStride;
+  hipLaunchKernelGGL(clear_u32_kernel, dim3(ceil_div(clear, kB)), dim3(kB), 0, s, g.cnt, clear);
+  hipLaunchKernelGGL(sil_pixel_list_kernel, dim3(ceil_div((long long)U * V, kB), (unsigned)(B * C)), dim3(kB), 0, s, a,
+                     g);
+  hipLaunchKernelGGL(sil_point_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, g);
+  hipLaunchKernelGGL(sil_grid_scan_kernel, dim3((unsigned)(B * C)), dim3(1024), 0, s, g);
   hipLaunchKernelGGL(sil_grid_scatter_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, g);
-  hipLaunchKernelGGL(sil_pixel_binned_kernel, dim3(ceil_div(PIX, kB)), dim3(kB), 0, s, a, g);
+  hipLaunchKernelGGL(sil_search_kernel, dim3(kSearchBlocks, (unsigned)(B * C)), dim3(kB), 0, s, a, g);
   return check_launch("dcx_mvsil_fwd(binned)");
 }
 
@@ -505,10 +653,10 @@ extern "C" dcx_status dcx_projected_mesh_boundary(const dcx_topo* topo, int B, i
   float* uv = (float*)workspace;
   unsigned char* cov = coverage ? coverage : (unsigned char*)workspace + align256(sizeof(float) * 2 * (size_t)B * C * N);
   const long long npix = (long long)B * C * H * W;
-  hipLaunchKernelGGL(fill_u8_kernel, dim3(ceil_div(npix, kB)), dim3(kB), 0, s, cov, npix);
+  hipLaunchKernelGGL(fill_u8_kernel, dim3(ceil_div(npix, 16 * kB)), dim3(kB), 0, s, cov, npix);
   hipLaunchKernelGGL(cov_project_kernel, dim3(ceil_div((long long)B * C * N, kB)), dim3(kB), 0, s, points, extrinsics,
                      intrinsics, B, C, N, uv);
-  hipLaunchKernelGGL(cov_raster_kernel, dim3(ceil_div((long long)B * C * F, kB)), dim3(kB), 0, s, uv, topo->faces, B,
+  hipLaunchKernelGGL(cov_raster_kernel, dim3(ceil_div((long long)B * C * F, kB / kCovLanes)), dim3(kB), 0, s, uv, topo->faces, B,
                      C, N, F, H, W, cov);
   hipLaunchKernelGGL(cov_boundary_kernel, dim3(ceil_div((long long)B * C * N, kB)), dim3(kB), 0, s, cov, uv, B, C, N,
                      H, W, is_boundary);

@@ -137,3 +137,58 @@ def test_projected_mesh_boundary_op_matches_oracle(near):
         assert (proj[np.isfinite(proj)] > 1e4).any()  # clamped projections of vertices behind a camera
     else:
         assert oflags.any() and not oflags.all()
+
+
+@pytest.mark.parametrize("U,V,N,scale,share,kind", [
+    (1, 1, 1, 2.0, 1.0, "contour"), (5, 3, 7, 3.0, 1.0, "contour"), (31, 29, 300, 1.0, 0.5, "noise"),
+    (64, 257, 2000, 0.01, 0.3, "contour"), (97, 30, 40, 40.0, 0.1, "noise"), (256, 60, 5000, 2.5, 0.02, "contour"),
+    (70, 70, 4000, 2.0, 1.0, "far"), (40, 50, 200, 2.0, 0.0, "noise"), (45, 45, 3000, 1.5, 1.0, "heap")])
+def test_grid_search_equals_the_scan_of_all_points(U, V, N, scale, share, kind):
+    """The same float distance and the same (distance, index) minimum, so the
+    outputs are the same bits: images with few and with many boundary pixels,
+    points around, beyond the radius of, and all in one cell of the grid."""
+    rng = np.random.default_rng(U * 1000 + V)
+    B, C = 2, 2
+    if kind == "noise":
+        dt = np.where(rng.uniform(size=(B, C, U, V)) < 0.6, 127, 90).astype(np.uint8)
+    else:
+        xx = np.arange(U * V).reshape(U, V) % U  # images are read as rows of U pixels
+        dt = np.broadcast_to(np.where(np.abs(xx - U // 2) <= 1, 127, 60).astype(np.uint8), (B, C, U, V)).copy()
+    crops = np.zeros((B, C, 7), np.float32)
+    crops[..., 0], crops[..., 2], crops[..., 3], crops[..., 4] = 1.5, scale, 20.0, -10.0
+    crops[..., 5], crops[..., 6] = 20.0 + U * scale, -10.0 + V * scale
+    lo, hi = crops[0, 0, 3:5], crops[0, 0, 5:7]
+    pts = (lo + (hi - lo) * rng.uniform(-0.3, 1.3, (B, C, N, 2))).astype(np.float32)
+    if kind == "far":
+        pts[..., 0] += 45 * scale
+    if kind == "heap":
+        pts = (lo + (hi - lo) * 0.4 + scale * rng.uniform(0, 0.5, (B, C, N, 2))).astype(np.float32)
+        pts[:, :, 1::2] = pts[:, :, ::2][:, :, :N // 2]  # ties
+    isb = (rng.uniform(size=(B, C, N)) < share).astype(np.uint8)
+    nrm = rng.normal(size=pts.shape).astype(np.float32)
+    args = [_t(pts), _t(nrm), _t(isb, torch.uint8), _t(dt, torch.uint8), _t(crops)]
+    for a, b in zip(silhouette.multi_view_silhouette_loss_gpu(*args, "binned"),
+                    silhouette.multi_view_silhouette_loss_gpu(*args, "brute")):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (7, 130), (65, 33)])
+def test_coverage_of_thin_huge_and_empty_triangles(H, W):
+    """Bit-exact against the oracle's divisions: triangles of no area, of a
+    few hundredths of a pixel, across the whole image, and on pixel centres."""
+    rng = np.random.default_rng(H)
+    ext = np.concatenate([np.eye(3), np.zeros((3, 1))], 1).reshape(1, 12).astype(np.float32)
+    intr = np.array([[1, 0, 0, 0, 1, 0, 0, 0, 1]], np.float32)  # a point (x, y, 1) is its pixel
+    tri = [rng.uniform(-5, [W + 5, H + 5], (3, 2)) for _ in range(60)]
+    tri += [rng.uniform(0, [W, H]) + rng.uniform(-s, s, (3, 2)) for s in (0.02, 0.5, 2.0, 1e4) for _ in range(30)]
+    tri += [np.repeat(rng.uniform(0, [W, H], (1, 2)), 3, 0), np.stack([np.zeros(2), [W, H], [2.0 * W, 2.0 * H]])]
+    tri += [np.array([[0.5, 0.5], [0.5 + k, 0.5], [0.5, 0.5 + k]]) for k in (1, 2, 8)]
+    xy = np.concatenate(tri)
+    V = np.concatenate([xy, np.ones((len(xy), 1))], 1)[None].astype(np.float32)
+    faces = np.arange(len(xy), dtype=np.int32).reshape(-1, 3)
+    for f in (faces, faces[:, ::-1].copy()):
+        flags, cov = silhouette.projected_mesh_boundary_gpu(_t(V), _t(ext), _t(intr), renderer.Topology(f, len(xy)),
+                                                            render_u=W, render_v=H, return_coverage=True)
+        proj, ocov = orc.mesh_coverage(f, V, ext, intr, H, W)
+        assert np.array_equal(cov.cpu().numpy(), ocov) and ocov.any()
+        assert np.array_equal(flags.cpu().numpy().astype(np.uint8), orc.boundary_flags(proj, ocov))
