@@ -22,6 +22,7 @@ SIGNATURES: dict[str, str] = {
     "dcx_dqs_fwd": "pppppiiiippppS",
     "dcx_dqs_bwd": "pppppppiiiipppiS",
     "dcx_dof_grad": "pppppiiiiipS",
+    "dcx_dof_grad_split": "pppppiiiiippzS",
     "dcx_lbs_fwd": "ppppppiiiippppS",
     "dcx_lbs_bwd": "ppppppiiiipppiS",
     "dcx_topo_create": "piipp",
@@ -61,14 +62,14 @@ SIGNATURES: dict[str, str] = {
 }
 
 # Functions whose return type is not dcx_status.
-_RESTYPES = {"dcx_render_workspace_size": ctypes.c_size_t, "dcx_ed_workspace_size": ctypes.c_size_t,
+_RESTYPES = {"dcx_dof_grad_workspace_size": ctypes.c_size_t, "dcx_render_workspace_size": ctypes.c_size_t, "dcx_ed_workspace_size": ctypes.c_size_t,
              "dcx_mvsil_workspace_size": ctypes.c_size_t, "dcx_pipeline_num_stages": ctypes.c_int,
              "dcx_pipeline_stage_name": ctypes.c_char_p, "dcx_normal_map_workspace_size": ctypes.c_size_t,
              "dcx_edt_workspace_size": ctypes.c_size_t, "dcx_dtloss_workspace_size": ctypes.c_size_t,
              "dcx_render_bwd_workspace_size": ctypes.c_size_t,
              "dcx_pipeline_tile_width": ctypes.c_int, "dcx_pipeline_grid_cap": ctypes.c_int,
              "dcx_projected_mesh_boundary_workspace_size": ctypes.c_size_t}
-_EXTRA_ARGTYPES = {"dcx_render_workspace_size": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int],
+_EXTRA_ARGTYPES = {"dcx_dof_grad_workspace_size": [ctypes.c_int] * 3, "dcx_render_workspace_size": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int],
                    "dcx_ed_workspace_size": [ctypes.c_void_p, ctypes.c_int],
                    "dcx_mvsil_workspace_size": [ctypes.c_int] * 5, "dcx_pipeline_num_stages": [],
                    "dcx_pipeline_stage_name": [ctypes.c_int],

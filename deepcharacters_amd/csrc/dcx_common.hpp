@@ -42,6 +42,29 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Sums of eight values over a wavefront (all lanes active): lane l gets the sum
+// of v[l & 7].  Each of the first three exchanges halves the values a lane
+// carries, so this is 10 exchanges where eight separate sums take 48.
+__device__ __forceinline__ float wave_sum8(const float* v) {
+  const int lane = threadIdx.x & 63;
+  float a[4], b[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // lanes 1 apart: keep v[2 i + bit 0]
+    const float keep = lane & 1 ? v[2 * i + 1] : v[2 * i], give = lane & 1 ? v[2 * i] : v[2 * i + 1];
+    a[i] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0xB1, 0xf, 0xf, false));
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // lanes 2 apart
+    const float keep = lane & 2 ? a[2 * i + 1] : a[2 * i], give = lane & 2 ? a[2 * i] : a[2 * i + 1];
+    b[i] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x4E, 0xf, 0xf, false));
+  }
+  const float keep = lane & 4 ? b[1] : b[0], give = lane & 4 ? b[0] : b[1];
+  float t = keep + __shfl_xor(give, 4, 64);
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+  return t;
+}
+
 // Smallest value of a group of 4, 16 or 64 lanes (all of them active), valid in
 // every lane: DPP row operations, which need no LDS crossbar round trip, and
 // for the whole wavefront the four rows' results through scalar registers.

@@ -62,41 +62,77 @@ __device__ __forceinline__ A34 a34_mul(const A34& a, const A34& b) {
   return r;
 }
 
-// One workgroup per pose: lane 0 walks the tree parents-first into LDS (the
-// chain is short and sequential), then the lanes write joint positions and
-// axes and the skinning transforms, as dual quaternions (out_dq) and/or as
-// rotation + translation (out_T, the linear-blend-skinning form).
+// A joint's transform in its parent's frame: T(offset) * M(value).
+__device__ __forceinline__ A34 fk_local(const SkelArgs& s, const float* dofs, int b, int j) {
+  const int dj = s.dof[j];
+  const float v = dj >= 0 ? dofs[(size_t)b * s.D + dj] : 0.f;
+  const float ax = s.axis[3 * j], ay = s.axis[3 * j + 1], az = s.axis[3 * j + 2];
+  const float ox = s.offset[3 * j], oy = s.offset[3 * j + 1], oz = s.offset[3 * j + 2];
+  if (s.type[j] != 0)
+    return {{1.f, 0.f, 0.f, ox + ax * v, 0.f, 1.f, 0.f, oy + ay * v, 0.f, 0.f, 1.f, oz + az * v}};
+  float sn, cs;
+  sincosf(v, &sn, &cs);
+  const float C = 1.f - cs;
+  return {{ax * ax * C + cs, ax * ay * C - az * sn, ax * az * C + ay * sn, ox,
+           ay * ax * C + az * sn, ay * ay * C + cs, ay * az * C - ax * sn, oy,
+           az * ax * C - ay * sn, az * ay * C + ax * sn, az * az * C + cs, oz}};
+}
+
+// One workgroup per pose.  The joints' global transforms come from pointer
+// doubling: every joint starts with its local transform and its parent, and
+// in each round multiplies by the transform of the joint it points to and
+// takes over that joint's pointer, so a chain of n joints needs log2(n)
+// rounds (a lane that walked the 57 joints of the body one after the other
+// took 30 us of loads and products; this takes 5).  Then the lanes write
+// joint positions and axes and the skinning transforms, as dual quaternions
+// (out_dq) and/or as rotation + translation (out_T, the
+// linear-blend-skinning form).  kPer: joints per lane.
+template <int kPer>
 __global__ __launch_bounds__(kFkBlock) void fk_kernel(SkelArgs s, const float* dofs, float* out_dq,
                                                        float* out_jpos, float* out_jaxis, float* out_T) {
-  __shared__ float s_g[kMaxFkJoints * 12];
+  __shared__ float s_g[kPer * kFkBlock * 12];
+  __shared__ short s_up[kPer * kFkBlock];
   const int b = blockIdx.x;
-  if (threadIdx.x == 0) {
-    for (int j = 0; j < s.J; ++j) {
-      const int dj = s.dof[j];
-      const float v = dj >= 0 ? dofs[(size_t)b * s.D + dj] : 0.f;
-      const float ax = s.axis[3 * j], ay = s.axis[3 * j + 1], az = s.axis[3 * j + 2];
-      const float ox = s.offset[3 * j], oy = s.offset[3 * j + 1], oz = s.offset[3 * j + 2];
-      A34 L;
-      if (s.type[j] == 0) {
-        float sn, cs;
-        sincosf(v, &sn, &cs);
-        const float C = 1.f - cs;
-        L = {{ax * ax * C + cs, ax * ay * C - az * sn, ax * az * C + ay * sn, ox,
-              ay * ax * C + az * sn, ay * ay * C + cs, ay * az * C - ax * sn, oy,
-              az * ax * C - ay * sn, az * ay * C + ax * sn, az * az * C + cs, oz}};
-      } else {
-        L = {{1.f, 0.f, 0.f, ox + ax * v, 0.f, 1.f, 0.f, oy + ay * v, 0.f, 0.f, 1.f, oz + az * v}};
-      }
-      A34 G = L;
-      if (s.parent[j] >= 0) {
-        A34 P;
-        for (int k = 0; k < 12; ++k) P.m[k] = s_g[12 * s.parent[j] + k];
-        G = a34_mul(P, L);
-      }
-      for (int k = 0; k < 12; ++k) s_g[12 * j + k] = G.m[k];
+  A34 G[kPer];
+  int up[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int j = i * kFkBlock + (int)threadIdx.x;
+    up[i] = -1;
+    if (j < s.J) {
+      G[i] = fk_local(s, dofs, b, j);
+      up[i] = s.parent[j];
     }
   }
-  __syncthreads();
+  for (;;) {
+    bool more = false;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int j = i * kFkBlock + (int)threadIdx.x;
+      more |= up[i] >= 0;
+      if (j < s.J) {
+        for (int k = 0; k < 12; ++k) s_g[12 * j + k] = G[i].m[k];
+        s_up[j] = (short)up[i];
+      }
+    }
+    if (!__syncthreads_or(more)) break;
+    A34 P[kPer];
+    int next[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      next[i] = -1;
+      if (up[i] >= 0) {
+        for (int k = 0; k < 12; ++k) P[i].m[k] = s_g[12 * up[i] + k];
+        next[i] = s_up[up[i]];
+      }
+    }
+    __syncthreads();  // all lanes have read this round's transforms
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      if (up[i] >= 0) G[i] = a34_mul(P[i], G[i]);
+      up[i] = next[i];
+    }
+  }
   for (int j = threadIdx.x; j < s.J; j += kFkBlock) {
     const float* g = s_g + 12 * j;
     const float ax = s.axis[3 * j], ay = s.axis[3 * j + 1], az = s.axis[3 * j + 2];
@@ -152,6 +188,16 @@ __global__ __launch_bounds__(kFkBlock) void fk_kernel(SkelArgs s, const float* d
     o[6] = 0.5f * (tx * q[1] - ty * q[0] + tz * q[3]);
     o[7] = -0.5f * (tx * q[0] + ty * q[1] + tz * q[2]);
   }
+}
+
+// A joint per lane, or as many as the largest skeleton needs.
+void launch_fk(const SkelArgs& a, int B, const float* dofs, float* dq, float* jpos, float* jaxis, float* T,
+               hipStream_t s) {
+  static_assert(kMaxFkJoints <= 4 * kFkBlock, "four joints a lane");
+  if (a.J <= kFkBlock)
+    hipLaunchKernelGGL(fk_kernel<1>, dim3(B), dim3(kFkBlock), 0, s, a, dofs, dq, jpos, jaxis, T);
+  else
+    hipLaunchKernelGGL(fk_kernel<4>, dim3(B), dim3(kFkBlock), 0, s, a, dofs, dq, jpos, jaxis, T);
 }
 
 // Pose2EmbeddedGraphCpu (Pose2EmbeddedGraphCPUOp.cpp:129-302) on the GPU: one
@@ -297,8 +343,7 @@ extern "C" dcx_status dcx_fk(const dcx_skeleton* s, int B, const float* dofs, fl
   DCX_REQUIRE(dual_quaternions && joint_pos && joint_axis, "dcx_fk: null output");
   const SkelArgs a{s->J, s->D, s->Js, s->parent, s->type, s->dof, s->offset, s->axis, s->skin_joint, s->skin_scale,
                    s->skin_bind};
-  hipLaunchKernelGGL(fk_kernel, dim3(B), dim3(kFkBlock), 0, as_stream(stream), a, dofs, dual_quaternions, joint_pos,
-                     joint_axis, (float*)nullptr);
+  launch_fk(a, B, dofs, dual_quaternions, joint_pos, joint_axis, nullptr, as_stream(stream));
   return check_launch("dcx_fk");
 }
 
@@ -309,8 +354,7 @@ extern "C" dcx_status dcx_fk_transforms(const dcx_skeleton* s, int B, const floa
   DCX_REQUIRE(transforms && joint_pos && joint_axis, "dcx_fk_transforms: null output");
   const SkelArgs a{s->J, s->D, s->Js, s->parent, s->type, s->dof, s->offset, s->axis, s->skin_joint, s->skin_scale,
                    s->skin_bind};
-  hipLaunchKernelGGL(fk_kernel, dim3(B), dim3(kFkBlock), 0, as_stream(stream), a, dofs, (float*)nullptr, joint_pos,
-                     joint_axis, transforms);
+  launch_fk(a, B, dofs, nullptr, joint_pos, joint_axis, transforms, as_stream(stream));
   return check_launch("dcx_fk_transforms");
 }
 

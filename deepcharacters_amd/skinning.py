@@ -86,8 +86,9 @@ def dof_grad(g_pos: torch.Tensor, skinned_pos: torch.Tensor, joint_pos: torch.Te
     inf = dev(influence, "influence")
     D, E = inf.shape[0], inf.shape[1]
     out = torch.empty((B, D), device=gp.device)
-    _lib.call("dcx_dof_grad", ptr(gp), ptr(sp), ptr(jp), ptr(ja), ptr(inf), B, N, Jall, D, E,
-              ptr(out), stream_ptr())
+    ws = torch.empty(_lib.load().dcx_dof_grad_workspace_size(B, D, E), dtype=torch.uint8, device=gp.device)
+    _lib.call("dcx_dof_grad_split", ptr(gp), ptr(sp), ptr(jp), ptr(ja), ptr(inf), B, N, Jall, D, E,
+              ptr(out), ptr(ws), ws.numel(), stream_ptr())
     return out
 
 

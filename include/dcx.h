@@ -100,6 +100,17 @@ dcx_status dcx_dof_grad(const float* g_pos, const float* skinned_pos, const floa
                         const float* joint_axis, const float* influence, int B, int N,
                         int Jall, int D, int max_entries, float* g_dofs, void* stream);
 
+/*
+ * dcx_dof_grad with each row split over workgroups and the influence table
+ * read once for several poses, for callers that have a workspace of
+ * dcx_dof_grad_workspace_size() bytes (4-byte aligned).
+ */
+size_t dcx_dof_grad_workspace_size(int B, int D, int max_entries);
+dcx_status dcx_dof_grad_split(const float* g_pos, const float* skinned_pos, const float* joint_pos,
+                              const float* joint_axis, const float* influence, int B, int N,
+                              int Jall, int D, int max_entries, float* g_dofs, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Linear blend skinning                                                    */
 /* ------------------------------------------------------------------------ */

@@ -115,3 +115,22 @@ def test_fk_rejects_bad_trees():
     from deepcharacters_amd import _lib
     with pytest.raises(_lib.DcxError):
         skinning.Skeleton(bad)
+
+
+@pytest.mark.parametrize("J,chain", [(1, True), (2, True), (255, True), (256, False), (257, True), (1024, False)])
+def test_fk_of_long_chains_and_large_trees(J, chain):
+    """One and four joints a lane, chains as long as the tree: a product of n
+    rotations in 32 bits is within about n 2^-23 of the exact one."""
+    rng = np.random.default_rng(J)
+    parent = np.arange(-1, J - 1) if chain else np.array([-1] + [int(rng.integers(0, j)) for j in range(1, J)])
+    skin = np.array([0, J // 2, J - 1], np.int32)
+    bind = np.tile(np.array([1, 0, 0, 0.1, 0, 1, 0, -0.2, 0, 0, 1, 0.3]), (3, 1))
+    desc = dict(parent=parent.astype(np.int32), type=rng.integers(0, 2, J).astype(np.int32),
+                dof=np.arange(J).astype(np.int32), offset=0.05 * rng.normal(size=(J, 3)),
+                axis=scenes.random_unit(rng, (J,)), skin_joint=skin, skin_scale=np.ones(3), skin_bind=bind, num_dofs=J)
+    dofs = rng.uniform(-0.5, 0.5, (3, J)).astype(np.float32)
+    dq, jp, ja = skinning.skeleton_fk(skinning.Skeleton(desc), _t(dofs))
+    rdq, rjp, rja = orc.fk(desc, dofs.astype(np.float64))
+    tol = 1e-6 + 2e-7 * J
+    assert _rel(_align(dq.cpu().numpy(), rdq), rdq) < tol
+    assert _rel(jp.cpu().numpy(), rjp) < tol and _rel(ja.cpu().numpy(), rja) < tol

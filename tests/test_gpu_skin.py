@@ -138,3 +138,60 @@ def test_autograd_matches_finite_differences_fp64_oracle():
         fd = (lp - lm) / (2 * h)
         got = float(t_dq.grad.reshape(-1)[i])
         assert abs(got - fd) <= 1e-4 * max(1.0, abs(fd)), (i, got, fd)
+
+
+@pytest.mark.parametrize("B,E,Jall", [(1, 1, 1), (8, 2048, 3), (9, 2049, 128), (3, 4500, 129), (17, 70, 5)])
+def test_split_dof_grad_at_the_edges_of_parts_poses_and_joints(B, E, Jall):
+    """Rows that end before, at and after the end of a part, with entries after
+    the end that name no vertex; the one-workgroup-a-row entry as well.  Sums
+    of up to E products of order 1 in 32 bits: within E * 2^-24 of their size."""
+    rng = np.random.default_rng(B * 1000 + E)
+    N, D = 300, 6
+    gp, sp = rng.normal(size=(B, N, 3)), rng.normal(size=(B, N, 3))
+    jp, ja = rng.normal(size=(B, Jall, 3)), scenes.random_unit(rng, (B, Jall))
+    infl = np.full((D, E, 4), 1e9)  # nothing behind a row's end may be read as a vertex
+    for d, m in enumerate([E, 0, min(E, 2048), min(E, 2047), E // 2, max(E - 1, 0)]):
+        infl[d, :m, 0] = rng.integers(0, N, m)
+        infl[d, :m, 1] = rng.integers(0, 2, m)
+        infl[d, :m, 2] = rng.integers(0, Jall, m)
+        infl[d, :m, 3] = rng.uniform(0, 1, m)
+        if m < E:
+            infl[d, m, 0] = -1
+    args = [_t(a) for a in (gp, sp, jp, ja, infl)]
+    out = skinning.dof_grad(*args)
+    ref = orc.dof_grad(*[a.cpu().numpy() for a in args])
+    one = torch.empty_like(out)
+    from deepcharacters_amd import _lib
+    _lib.call("dcx_dof_grad", *[a.data_ptr() for a in args], B, N, Jall, D, E, one.data_ptr(),
+              torch.cuda.current_stream().cuda_stream)
+    for got in (out, one):
+        assert np.abs(got.cpu().numpy() - ref).max() <= 4e-6 * max(1.0, np.sqrt(E))
+
+
+@pytest.mark.parametrize("N,J,K,order", [(1, 1, 4, "one"), (64, 5, 4, "few"), (257, 256, 4, "random"),
+                                         (300, 257, 4, "random"), (1000, 40, 3, "random"), (513, 30, 8, "random")])
+def test_joint_gradients_of_ordered_and_unordered_skinnings(N, J, K, order):
+    """Few joints a wavefront (summed in registers), more than it goes through
+    (the rest added one by one), more than LDS holds; sums of about N K / J
+    products in 32 bits."""
+    rng = np.random.default_rng(N + J)
+    B = 2
+    ji = {"one": np.zeros((N, K)), "few": np.arange(N)[:, None] // 40 + np.arange(K) % 3,
+          "random": rng.integers(0, J, (N, K))}[order].astype(np.int32) % J
+    dq = scenes.random_joint_dqs(rng, rng.normal(size=(J, 3)), B, 0.4)
+    w, v, g = rng.uniform(0.1, 1, (B, N, K)), rng.normal(size=(N, 3)), rng.normal(size=(B, N, 3))
+    g_dq, g_w, g_r = skinning.dq_skinning_backward(_t(g), _t(dq), _t(w), _t(ji, torch.int32), _t(v), need_rest=True)
+    o_dq, o_w, o_r = orc.dqs_bwd(g, dq, w, ji, v)
+    assert _rel(g_dq.cpu(), o_dq) < 1e-4 and _rel(g_r.cpu(), o_r) < 1e-5
+    # a weight's gradient is a dot product with the joint's gradient, exactly 0
+    # where one joint has all the weight: its rounding is relative to the factors
+    assert np.abs(g_w.cpu().numpy() - o_w).max() < 1e-5 * max(np.abs(o_w).max(), np.abs(o_dq).max())
+    tr, disp = rng.normal(size=(B, J, 12)), 0.01 * rng.normal(size=(B, N, 3))
+    g_w, g_d, g_t = skinning.lb_skinning_backward(_t(g), _t(tr), _t(w), _t(ji, torch.int32), _t(v), _t(disp))
+    o_w, o_d, o_t = orc.lbs_bwd(g, tr, w, ji, v, disp)
+    assert _rel(g_t.cpu(), o_t) < 1e-4 and _rel(g_w.cpu(), o_w) < 1e-5 and _rel(g_d.cpu(), o_d) < 1e-5
+    # an infinite gradient of one vertex reaches its own joints only
+    g[0, 0] = np.inf
+    got = skinning.dq_skinning_backward(_t(g), _t(dq), _t(w), _t(ji, torch.int32), _t(v))[0].cpu().numpy()
+    mine = np.isin(np.arange(J), ji[0])
+    assert np.isfinite(got[1]).all() and np.isfinite(got[0][~mine]).all() and not np.isfinite(got[0][mine]).all()
