@@ -1,10 +1,11 @@
 // Rasterizer forward on gfx950: topology, the plain path (the reference's
 // launch decomposition: host loop over batch elements, one lane per
 // (camera, face) walking its bounding box with global 64-bit atomicMin) and
-// the binned path (all batch elements and views in one launch sequence:
-// triangle setup + tile binning, then one workgroup per 32x8 screen tile
-// resolving depth in LDS with 64-bit ds_min on packed (depth, face) keys and
-// writing every output pixel exactly once, coalesced).
+// the binned path (all batch elements and views in one launch sequence of
+// five: projections and face normals; vertex normals and tile counts; list
+// offsets; tile lists; then one workgroup per 32x8 screen tile resolving
+// depth in LDS with 64-bit ds_min on packed (depth, face) keys and writing
+// every output pixel exactly once, coalesced).
 #include <mutex>
 #include <vector>
 
@@ -57,11 +58,9 @@ dcx_status topo_create(const int32_t* faces, int F, int N, const float* tc, dcx_
 
 constexpr int kB = 256;
 
-__global__ __launch_bounds__(kB) void project_kernel(const float* __restrict__ vpos,
-                                                      const float* __restrict__ ext,
-                                                      const float* __restrict__ intr, int N, int C,
-                                                      int views, f4* __restrict__ proj) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
+__device__ __forceinline__ void project_one(const float* __restrict__ vpos, const float* __restrict__ ext,
+                                            const float* __restrict__ intr, int N, int C, int views, long long i,
+                                            f4* __restrict__ proj) {
   if (i >= (long long)views * N) return;
   const int view = (int)(i / N), v = (int)(i - (long long)view * N);
   const int b = view / C;
@@ -71,10 +70,15 @@ __global__ __launch_bounds__(kB) void project_kernel(const float* __restrict__ v
   proj[i] = project_vertex(E, K, vpos + ((size_t)b * N + v) * 3);
 }
 
-__global__ __launch_bounds__(kB) void face_normal_kernel(const float* __restrict__ vpos,
-                                                          const int* __restrict__ faces, int N, int F,
-                                                          int B, float* __restrict__ fn) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
+__global__ __launch_bounds__(kB) void project_kernel(const float* __restrict__ vpos,
+                                                      const float* __restrict__ ext,
+                                                      const float* __restrict__ intr, int N, int C,
+                                                      int views, f4* __restrict__ proj) {
+  project_one(vpos, ext, intr, N, C, views, (long long)blockIdx.x * kB + threadIdx.x, proj);
+}
+
+__device__ __forceinline__ void face_normal_one(const float* __restrict__ vpos, const int* __restrict__ faces, int N,
+                                                int F, int B, long long i, float* __restrict__ fn) {
   if (i >= (long long)B * F) return;
   const int b = (int)(i / F), f = (int)(i - (long long)b * F);
   const float* vp = vpos + (size_t)b * N * 3;
@@ -84,28 +88,67 @@ __global__ __launch_bounds__(kB) void face_normal_kernel(const float* __restrict
   fn[3 * i] = n.x; fn[3 * i + 1] = n.y; fn[3 * i + 2] = n.z;
 }
 
+__global__ __launch_bounds__(kB) void face_normal_kernel(const float* __restrict__ vpos,
+                                                          const int* __restrict__ faces, int N, int F,
+                                                          int B, float* __restrict__ fn) {
+  face_normal_one(vpos, faces, N, F, B, (long long)blockIdx.x * kB + threadIdx.x, fn);
+}
+
 // Sum of face normals over each vertex's faces (increasing face order);
-// also broadcast into the [B,C,N,3] vertex_normal output when given.
+// also broadcast into the [B,C,N,3] vertex_normal output when given.  A
+// vertex's loads are issued eight at a time; the few vertices with more than
+// kManyFaces faces (the poles of a mesh: a hundred and more) are loaded by the
+// whole wavefront and added up in the same order, since a lane that walks such
+// a list load by load is the last of the launch (24 us of 24 for 50k vertices
+// and 8 views; MEASUREDVN).  All lanes of a wavefront call it.
+constexpr int kManyFaces = 16;
+__device__ __forceinline__ void vertex_normal_one(const float* __restrict__ fn, const int* __restrict__ off,
+                                                  const int* __restrict__ lst, int N, int F, int B, int C,
+                                                  long long i, float* __restrict__ vn, float* __restrict__ vn_out) {
+  const bool in = i < (long long)B * N;
+  const int b = in ? (int)(i / N) : 0, v = in ? (int)(i - (long long)b * N) : 0;
+  const float* fb = fn + (size_t)b * F * 3;
+  const int k0 = in ? off[v] : 0, k1 = in ? off[v + 1] : 0;
+  f3 s = mk3(0.f, 0.f, 0.f);
+  if (k1 - k0 <= kManyFaces)
+    for (int k = k0; k < k1; k += 8) {
+      f3 n[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) n[j] = ld3(fb + 3 * lst[min(k + j, k1 - 1)]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (k + j < k1) s = s + n[j];
+    }
+  for (unsigned long long many = __ballot(k1 - k0 > kManyFaces); many; many &= many - 1) {
+    const int src = __ffsll(many) - 1, lane = threadIdx.x & 63;
+    const int c0 = __builtin_amdgcn_readlane(k0, src), c1 = __builtin_amdgcn_readlane(k1, src);
+    const float* cb = fn + (size_t)__builtin_amdgcn_readlane(b, src) * F * 3;
+    f3 t = mk3(0.f, 0.f, 0.f);
+    for (int k = c0; k < c1; k += 64) {
+      const f3 n = ld3(cb + 3 * lst[min(k + lane, c1 - 1)]);
+      const int m = min(64, c1 - k);
+      for (int j = 0; j < m; ++j)
+        t = t + mk3(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.x), j)),
+                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.y), j)),
+                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.z), j)));
+    }
+    if (lane == src) s = t;
+  }
+  if (!in) return;
+  vn[3 * i] = s.x; vn[3 * i + 1] = s.y; vn[3 * i + 2] = s.z;
+  if (vn_out)
+    for (int c = 0; c < C; ++c) {
+      float* o = vn_out + (((size_t)b * C + c) * N + v) * 3;
+      o[0] = s.x; o[1] = s.y; o[2] = s.z;
+    }
+}
+
 __global__ __launch_bounds__(kB) void vertex_normal_kernel(const float* __restrict__ fn,
                                                             const int* __restrict__ off,
                                                             const int* __restrict__ lst, int N, int F,
                                                             int B, int C, float* __restrict__ vn,
                                                             float* __restrict__ vn_out) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)B * N) return;
-  const int b = (int)(i / N), v = (int)(i - (long long)b * N);
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-  const float* fb = fn + (size_t)b * F * 3;
-  for (int k = off[v]; k < off[v + 1]; ++k) {
-    const float* n = fb + 3 * lst[k];
-    s0 += n[0]; s1 += n[1]; s2 += n[2];
-  }
-  vn[3 * i] = s0; vn[3 * i + 1] = s1; vn[3 * i + 2] = s2;
-  if (vn_out)
-    for (int c = 0; c < C; ++c) {
-      float* o = vn_out + (((size_t)b * C + c) * N + v) * 3;
-      o[0] = s0; o[1] = s1; o[2] = s2;
-    }
+  vertex_normal_one(fn, off, lst, N, F, B, C, (long long)blockIdx.x * kB + threadIdx.x, vn, vn_out);
 }
 
 // Reference rule (uv2barycentric / rayTriangleIntersect, RendererUtil.h:26-128,
@@ -328,13 +371,6 @@ __global__ __launch_bounds__(kB) void clear_keys_kernel(unsigned long long* keys
   if (i < n) keys[i] = kEmptyKey;
 }
 
-// Zero fill of a counter array (a kernel rather than a memset, so that a
-// caller may capture the forward into a graph).
-__global__ __launch_bounds__(kB) void clear_u32_kernel(unsigned int* a, long long n) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i < n) a[i] = 0u;
-}
-
 // One lane per (camera, face): walks the triangle's pixel range and folds
 // its keys into the global depth buffer with 64-bit atomicMin.
 __global__ __launch_bounds__(kB) void raster_plain_kernel(RenderArgs a, int b, unsigned long long* keys) {
@@ -372,152 +408,276 @@ __global__ __launch_bounds__(kB) void resolve_plain_kernel(RenderArgs a, int b, 
 // Binned path
 // ---------------------------------------------------------------------------
 
-// Per (view, face): triangle record + number of tiles it touches.
-__global__ __launch_bounds__(kB) void tri_setup_count_kernel(RenderArgs a, BinArgs g) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)g.views * a.F) return;
-  const int view = (int)(i / a.F), f = (int)(i - (long long)view * a.F);
-  const f4* pv = a.proj + (size_t)view * a.N;
-  TriRec t;
-  if (!setup_tri(pv[a.faces[3 * f]], pv[a.faces[3 * f + 1]], pv[a.faces[3 * f + 2]], f, a.W, a.H, t)) {
-    t.bx0_by0 = 0x7fff7fff;  // empty range
-    t.bx1_by1 = 0;
-    g.tri[i] = t;
+// Launch 1: a lane per (view, vertex) projects, one per (batch element, face)
+// takes the face normal, and all of them clear the tile counts.
+__global__ __launch_bounds__(kB) void bin_prepare_kernel(RenderArgs a, BinArgs g, unsigned project_blocks, int B,
+                                                         float* fnrm) {
+  const long long id = (long long)blockIdx.x * kB + threadIdx.x;
+  for (long long t = id; t < g.tiles + 2; t += (long long)gridDim.x * kB) g.tile_cnt[t] = 0u;  // and the totals
+  if (blockIdx.x < project_blocks)
+    project_one(a.vpos, a.ext, a.intr, a.N, a.C, g.views, id, a.proj);
+  else
+    face_normal_one(a.vpos, a.faces, a.N, a.F, B, id - (long long)project_blocks * kB, fnrm);
+}
+
+// Adds to the counters of the wavefront's tiles (lanes with `active`), one
+// atomic a distinct tile, and returns each lane's own place: neighbouring
+// faces fall into the same few tiles, and the atomics are what the binning
+// costs (an atomic per (face, tile) made the two passes 320 and 375 us for
+// 16 views of 200k faces at 2048 x 2048; 78 and 92 now).  Faces without such order are left to
+// atomics of their own after kTileRounds tiles.  All lanes of a wavefront call
+// it.
+constexpr int kTileRounds = 16;
+template <bool kPlace>
+__device__ __forceinline__ unsigned int tile_add(unsigned int* ctr, bool active, unsigned int tile) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long mine = 1ull << lane;
+  unsigned long long left = __ballot(active);
+  for (int r = 0; left && r < kTileRounds; ++r) {
+    const unsigned int t = (unsigned int)__builtin_amdgcn_readlane((int)tile, __ffsll(left) - 1);
+    const unsigned long long same = __ballot(active && tile == t);
+    if (active && tile == t) mine = same;
+    left &= ~same;
+  }
+  const int first = active ? __ffsll(mine) - 1 : lane;
+  unsigned int base = 0;
+  if (active && lane == first) base = atomicAdd(ctr + tile, (unsigned int)__popcll(mine));
+  if (!kPlace) return 0;
+  return (unsigned int)__shfl((int)base, first, 64) + (unsigned int)__popcll(mine & ((1ull << lane) - 1ull));
+}
+
+// Calls f(active, tile, face, shared) for every (face, tile) pair of the
+// wavefront: a lane's own tiles one after the other (shared: lanes may have
+// the same one), a face over more than kManyTiles by all lanes, a tile each.
+// r: first and last tile of the lane's face (x | y << 16), first >
+// last x for none.
+constexpr int kManyTiles = 16;
+template <class Fn>
+__device__ __forceinline__ void for_tiles(uint2 r, int tiles_x, unsigned int view_base, int face, Fn f) {
+  const int x0 = r.x & 0xffff, y0 = r.x >> 16, x1 = r.y & 0xffff, y1 = r.y >> 16;
+  const int nx = x1 - x0 + 1, n = nx > 0 ? nx * (y1 - y0 + 1) : 0;
+  int x = x0, y = y0;
+  for (int k = 0; __ballot(n <= kManyTiles && k < n); ++k) {
+    f(n <= kManyTiles && k < n, view_base + (unsigned int)(y * tiles_x + x), face, true);
+    if (++x > x1) { x = x0; ++y; }
+  }
+  for (unsigned long long many = __ballot(n > kManyTiles); many; many &= many - 1) {
+    const int src = __ffsll(many) - 1;
+    const int bx = __builtin_amdgcn_readlane(x0, src), by = __builtin_amdgcn_readlane(y0, src);
+    const int bw = __builtin_amdgcn_readlane(nx, src), bn = __builtin_amdgcn_readlane(n, src);
+    const unsigned int base = (unsigned int)__builtin_amdgcn_readlane((int)view_base, src);
+    const int bf = __builtin_amdgcn_readlane(face, src);
+    for (int k0 = 0; k0 < bn; k0 += 64) {
+      const int k = k0 + (int)(threadIdx.x & 63);
+      f(k < bn, base + (unsigned int)((by + k / bw) * tiles_x + bx + k % bw), bf, false);
+    }
+  }
+}
+
+// Launch 2: vertex normals, and per (view, face) the range of tiles it touches
+// and their counts.
+__global__ __launch_bounds__(kB) void bin_count_kernel(RenderArgs a, BinArgs g, unsigned normal_blocks, int B,
+                                                       const float* fnrm, const int* vf_off, const int* vf_list,
+                                                       float* vnrm, float* vn_out) {
+  if (blockIdx.x < normal_blocks) {
+    vertex_normal_one(fnrm, vf_off, vf_list, a.N, a.F, B, a.C, (long long)blockIdx.x * kB + threadIdx.x, vnrm, vn_out);
     return;
   }
-  g.tri[i] = t;
-  const int x0 = t.bx0_by0 & 0xffff, y0 = t.bx0_by0 >> 16, x1 = t.bx1_by1 & 0xffff, y1 = t.bx1_by1 >> 16;
-  unsigned int* cnt = g.tile_cnt + (size_t)view * g.tiles_per_view;
-  for (int ty = y0 / kTileH; ty <= y1 / kTileH; ++ty)
-    for (int tx = x0 / kTileW; tx <= x1 / kTileW; ++tx) atomicAdd(cnt + ty * g.tiles_x + tx, 1u);
-}
-
-__global__ __launch_bounds__(kB) void bin_scatter_kernel(RenderArgs a, BinArgs g) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)g.views * a.F) return;
-  const TriRec& t = g.tri[i];
-  if (t.bx0_by0 == 0x7fff7fff) return;
-  const int view = (int)(i / a.F);
-  const int x0 = t.bx0_by0 & 0xffff, y0 = t.bx0_by0 >> 16, x1 = t.bx1_by1 & 0xffff, y1 = t.bx1_by1 >> 16;
-  const size_t base = (size_t)view * g.tiles_per_view;
-  for (int ty = y0 / kTileH; ty <= y1 / kTileH; ++ty)
-    for (int tx = x0 / kTileW; tx <= x1 / kTileW; ++tx) {
-      const size_t tile = base + ty * g.tiles_x + tx;
-      const unsigned int slot = g.tile_off[tile] + atomicAdd(g.tile_fill + tile, 1u);
-      if (slot < g.capacity) g.bins[slot] = (unsigned int)i;
-    }
-}
-
-__device__ __forceinline__ void raster_tri_in_tile(const TriRec& t, int tx0, int ty0,
-                                                   unsigned long long* s_key) {
-  const int x0 = max(t.bx0_by0 & 0xffff, tx0), y0 = max(t.bx0_by0 >> 16, ty0);
-  const int x1 = min(t.bx1_by1 & 0xffff, tx0 + kTileW - 1), y1 = min(t.bx1_by1 >> 16, ty0 + kTileH - 1);
-  if (x0 > x1 || y0 > y1) return;
-  EdgeWalk w;
-  w.init(t, x0, y0);
-  const int face = t.face_flags & kFaceMask;
-  long long row[3] = {w.e[0], w.e[1], w.e[2]};
-  for (int y = y0; y <= y1; ++y) {
-    long long e[3] = {row[0], row[1], row[2]};
-    for (int x = x0; x <= x1; ++x) {
-      if (w.inside(e))
-        atomicMin(s_key + (y - ty0) * kTileW + (x - tx0), make_key(interp_iz(e[0], e[1], e[2], t.iz), face));
-      e[0] += w.dx[0]; e[1] += w.dx[1]; e[2] += w.dx[2];
-    }
-    row[0] += w.dy[0]; row[1] += w.dy[1]; row[2] += w.dy[2];
+  const long long i = (long long)(blockIdx.x - normal_blocks) * kB + threadIdx.x;
+  uint2 r = make_uint2(1u, 0u);
+  int view = 0, f = 0;
+  if (i < (long long)g.views * a.F) {
+    view = (int)(i / a.F);
+    f = (int)(i - (long long)view * a.F);
+    const f4* pv = a.proj + (size_t)view * a.N;
+    TriRec t;
+    if (setup_tri(pv[a.faces[3 * f]], pv[a.faces[3 * f + 1]], pv[a.faces[3 * f + 2]], f, a.W, a.H, t))
+      r = make_uint2((unsigned)((t.bx0_by0 & 0xffff) / kTileW) | (unsigned)((t.bx0_by0 >> 16) / kTileH) << 16,
+                     (unsigned)((t.bx1_by1 & 0xffff) / kTileW) | (unsigned)((t.bx1_by1 >> 16) / kTileH) << 16);
+    g.range[i] = r;
   }
+  for_tiles(r, g.tiles_x, (unsigned)view * (unsigned)g.tiles_per_view, f,
+            [&](bool active, unsigned tile, int, bool shared) {
+              if (shared) tile_add<false>(g.tile_cnt, active, tile);
+              else if (active) atomicAdd(g.tile_cnt + tile, 1u);
+            });
 }
 
-// One workgroup per 32x8 tile.  Triangle-parallel raster into LDS keys, then
-// pixel-parallel resolve.  A tile whose list did not fit the bin capacity
-// scans every triangle of its view instead (slow, exact).
-__global__ __launch_bounds__(kTilePix) void fine_raster_kernel(RenderArgs a, BinArgs g) {
-  __shared__ unsigned long long s_key[kTilePix];
-  const int tile = blockIdx.x;
-  const int view = tile / g.tiles_per_view;
-  const int lt = tile - view * g.tiles_per_view;
-  const int tx0 = (lt % g.tiles_x) * kTileW, ty0 = (lt / g.tiles_x) * kTileH;
-  s_key[threadIdx.x] = kEmptyKey;
-  __syncthreads();
-  const unsigned int off = g.tile_off[tile], end = g.tile_off[tile + 1];
-  if (end <= g.capacity) {
-    for (unsigned int k = off + threadIdx.x; k < end; k += kTilePix) raster_tri_in_tile(g.tri[g.bins[k]], tx0, ty0, s_key);
-  } else {
-    const TriRec* tv = g.tri + (size_t)view * a.F;
-    for (int f = threadIdx.x; f < a.F; f += kTilePix) raster_tri_in_tile(tv[f], tx0, ty0, s_key);
+// Launch 3: every tile's place in the lists (in the order in which the
+// workgroups arrive; which part of the storage holds a tile's list changes no
+// result), and the tiles that have a list.  tile_cnt[tiles] and [tiles + 1]
+// are the totals of both.
+__global__ __launch_bounds__(kB) void bin_offset_kernel(BinArgs g) {
+  __shared__ unsigned long long s_wave[kB / 64];
+  __shared__ unsigned int s_base[2];
+  const long long t0 = ((long long)blockIdx.x * kB + threadIdx.x) * 4;
+  unsigned int c[4];
+  unsigned long long sum = 0;  // entries, and in the upper half tiles
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    c[k] = t0 + k < g.tiles ? g.tile_cnt[t0 + k] : 0u;
+    sum += c[k] ? (1ull << 32) + c[k] : 0ull;
   }
-  __syncthreads();
-  const int x = tx0 + (threadIdx.x % kTileW), y = ty0 + (threadIdx.x / kTileW);
-  if (x < a.W && y < a.H) resolve_pixel(a, view / a.C, view, x, y, s_key[threadIdx.x]);
-}
-
-// ---------------------------------------------------------------------------
-// Exclusive scan of the per-tile counts (three phases, 1024 elements/block).
-// ---------------------------------------------------------------------------
-
-__device__ __forceinline__ unsigned int block_exclusive_scan(unsigned int v, unsigned int* s_wave,
-                                                             unsigned int& total) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  unsigned int inc = v;
+  unsigned long long inc = sum;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const unsigned int o = __shfl_up(inc, d, 64);
+    const unsigned long long o = __shfl_up(inc, d, 64);
     if (lane >= d) inc += o;
   }
   if (lane == 63) s_wave[wid] = inc;
   __syncthreads();
-  unsigned int wave_base = 0;
-  total = 0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-    if (w < wid) wave_base += s_wave[w];
+  unsigned long long before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kB / 64; ++w) {
+    before += w < wid ? s_wave[w] : 0ull;
     total += s_wave[w];
   }
+  if (threadIdx.x < 2 && total)
+    s_base[threadIdx.x] = atomicAdd(g.tile_cnt + g.tiles + threadIdx.x, (unsigned int)(total >> (32 * threadIdx.x)));
   __syncthreads();
-  return wave_base + inc - v;
+  before += inc - sum;
+  unsigned int at = s_base[0] + (unsigned int)before, q = s_base[1] + (unsigned int)(before >> 32);
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (c[k]) {
+      g.tile_end[t0 + k] = at;
+      at += c[k];
+      g.full[q++] = (unsigned int)(t0 + k);
+    }
 }
 
-__global__ __launch_bounds__(256) void scan_blocks_kernel(const unsigned int* in, unsigned int* out,
-                                                          unsigned int* aux, long long n) {
-  __shared__ unsigned int s_wave[4];
-  const long long base = (long long)blockIdx.x * 1024 + threadIdx.x * 4;
-  unsigned int v[4], s = 0;
-  for (int k = 0; k < 4; ++k) { v[k] = base + k < n ? in[base + k] : 0u; s += v[k]; }
-  unsigned int total;
-  unsigned int ex = block_exclusive_scan(s, s_wave, total);
-  for (int k = 0; k < 4; ++k) {
-    if (base + k < n) out[base + k] = ex;
-    ex += v[k];
+// Launch 4: the face ids into the lists; a tile's cursor ends at its list's end.
+__global__ __launch_bounds__(kB) void bin_scatter_kernel(RenderArgs a, BinArgs g) {
+  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
+  const bool in = i < (long long)g.views * a.F;
+  const int view = in ? (int)(i / a.F) : 0;
+  for_tiles(in ? g.range[i] : make_uint2(1u, 0u), g.tiles_x, (unsigned)view * (unsigned)g.tiles_per_view,
+            (int)(i - (long long)view * a.F), [&](bool active, unsigned tile, int f, bool shared) {
+              unsigned int slot = 0;
+              if (shared) slot = tile_add<true>(g.tile_end, active, tile);
+              else if (active) slot = atomicAdd(g.tile_end + tile, 1u);
+              if (active && slot < g.capacity) g.bins[slot] = (unsigned int)f;
+            });
+}
+
+// Rows y0 + sub, y0 + sub + step, ... of a triangle's box in the tile.  The
+// edge values at a pixel centre of the box are below 2^29 where the triangle
+// is at most 64 pixels wide and high (factors below 2^15), so such triangles
+// are walked in 32 bits: the same whole numbers, a third of the instructions.
+__device__ __forceinline__ void raster_tri_in_tile(const TriRec& t, int tx0, int ty0, int sub, int step,
+                                                   unsigned long long* s_key) {
+  const int x0 = max(t.bx0_by0 & 0xffff, tx0), y0 = max(t.bx0_by0 >> 16, ty0);
+  const int x1 = min(t.bx1_by1 & 0xffff, tx0 + kTileW - 1), y1 = min(t.bx1_by1 >> 16, ty0 + kTileH - 1);
+  if (x0 > x1 || y0 + sub > y1) return;
+  const int face = t.face_flags & kFaceMask;
+  const int w = max(t.X[0], max(t.X[1], t.X[2])) - min(t.X[0], min(t.X[1], t.X[2]));
+  const int h = max(t.Y[0], max(t.Y[1], t.Y[2])) - min(t.Y[0], min(t.Y[1], t.Y[2]));
+  if (max(w, h) <= 64 * kSub) {
+    const int sg = (t.face_flags & (1 << 28)) ? -1 : 1;
+    const int cx = x0 * kSub + kSub / 2;
+    int ax[3], ay[3], bias[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int j = i == 2 ? 0 : i + 1, k = i == 0 ? 2 : i - 1;
+      ax[i] = (t.X[k] - t.X[j]) * sg;
+      ay[i] = (t.Y[k] - t.Y[j]) * sg;
+      bias[i] = (t.face_flags >> (29 + i)) & 1 ? -1 : 0;
+    }
+    for (int y = y0 + sub; y <= y1; y += step) {
+      const int cy = y * kSub + kSub / 2;
+      int e[3];  // with the tie rule's bias
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int j = i == 2 ? 0 : i + 1;
+        e[i] = __mul24(ax[i], cy - t.Y[j]) - __mul24(ay[i], cx - t.X[j]) + bias[i];
+      }
+      unsigned long long* row = s_key + (y - ty0) * kTileW - tx0;
+      for (int x = x0; x <= x1; ++x) {
+        if ((e[0] | e[1] | e[2]) >= 0) {
+          const float izp = (float)(e[0] - bias[0]) * t.iz[0] + (float)(e[1] - bias[1]) * t.iz[1] +
+                            (float)(e[2] - bias[2]) * t.iz[2];
+          atomicMin(row + x, make_key(izp, face));
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) e[i] -= ay[i] * kSub;
+      }
+    }
+    return;
   }
-  if (threadIdx.x == 0) aux[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(1024) void scan_aux_kernel(unsigned int* aux, int nb, unsigned int* total_out) {
-  __shared__ unsigned int s_wave[16];
-  unsigned int v[4], s = 0;
-  for (int k = 0; k < 4; ++k) { const int i = threadIdx.x * 4 + k; v[k] = i < nb ? aux[i] : 0u; s += v[k]; }
-  unsigned int total;
-  unsigned int ex = block_exclusive_scan(s, s_wave, total);
-  for (int k = 0; k < 4; ++k) {
-    const int i = threadIdx.x * 4 + k;
-    if (i < nb) aux[i] = ex;
-    ex += v[k];
+  EdgeWalk ew;
+  ew.init(t, x0, y0 + sub);
+  long long row[3] = {ew.e[0], ew.e[1], ew.e[2]};
+  for (int y = y0 + sub; y <= y1; y += step) {
+    long long e[3] = {row[0], row[1], row[2]};
+    for (int x = x0; x <= x1; ++x) {
+      if (ew.inside(e))
+        atomicMin(s_key + (y - ty0) * kTileW + (x - tx0), make_key(interp_iz(e[0], e[1], e[2], t.iz), face));
+      e[0] += ew.dx[0]; e[1] += ew.dx[1]; e[2] += ew.dx[2];
+    }
+    row[0] += ew.dy[0] * step; row[1] += ew.dy[1] * step; row[2] += ew.dy[2] * step;
   }
-  if (threadIdx.x == 0) *total_out = total;
 }
 
-__global__ __launch_bounds__(256) void scan_add_kernel(unsigned int* out, const unsigned int* aux, long long n) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] += aux[i / 1024];
-}
-
-dcx_status exclusive_scan(const unsigned int* in, unsigned int* out, unsigned int* aux, long long n,
-                          hipStream_t s) {
-  const int nb = (int)ceil_div(n, 1024);
-  DCX_REQUIRE(nb <= 4096, "scan of %lld elements exceeds 4M", n);
-  hipLaunchKernelGGL(scan_blocks_kernel, dim3(nb), dim3(256), 0, s, in, out, aux, n);
-  hipLaunchKernelGGL(scan_aux_kernel, dim3(1), dim3(1024), 0, s, aux, nb, out + n);
-  hipLaunchKernelGGL(scan_add_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, out, aux, n);
-  return check_launch("exclusive_scan");
+// Launch 5: kFineBlocks workgroups, as many as the chip holds, take the tiles
+// that have lists in turn.  Triangle-parallel raster into LDS keys (the
+// records are set up again from the projections: a stored one is 48 bytes
+// written and read), then pixel-parallel resolve.  With a short list, 2, 4 or 8
+// lanes share a triangle's rows.  A tile whose list did not fit the bin
+// capacity scans every triangle of its view instead (slow, exact).  Between
+// tiles a workgroup writes the background of eight tiles of a row, stores that
+// nothing waits for while the next tile's lists and vertices are loaded; a
+// workgroup for every tile, most of them background, kept under three
+// wavefronts a SIMD busy.  16 views of 2048 x 2048: 1,402 us at first, 973 with
+// 32-bit walks, 640 so (writing the images alone takes 320).
+constexpr int kFineBlocks = 256 * 6;
+constexpr int kBackTiles = kB / kTileW;  // tiles of one background piece: a pixel column a lane
+__global__ __launch_bounds__(kTilePix) void fine_raster_kernel(RenderArgs a, BinArgs g) {
+  __shared__ unsigned long long s_key[kTilePix];
+  const unsigned int full = g.tile_cnt[g.tiles + 1];
+  const int tiles_y = g.tiles_per_view / g.tiles_x, chunks = (g.tiles_x + kBackTiles - 1) / kBackTiles;
+  const unsigned int pieces = (unsigned int)g.views * tiles_y * chunks;
+  for (unsigned int q = blockIdx.x; q < full || q < pieces; q += gridDim.x) {
+    // the background piece's pixel column, and whether its tile is empty
+    int bview = 0, by = 0, bx = 0;
+    bool back = false;
+    if (q < pieces) {
+      const int strip = (int)(q / chunks);
+      bview = strip / tiles_y;
+      by = (strip - bview * tiles_y) * kTileH;
+      bx = (int)(q - (unsigned int)strip * chunks) * kB + (int)threadIdx.x;
+      back = bx < a.W && g.tile_cnt[(size_t)strip * g.tiles_x + bx / kTileW] == 0;
+    }
+    if (q < full) {
+      const unsigned int tile = g.full[q];
+      const int view = (int)(tile / g.tiles_per_view), lt = (int)(tile - (unsigned int)view * g.tiles_per_view);
+      const int ty0 = lt / g.tiles_x * kTileH, tx0 = lt % g.tiles_x * kTileW;
+      const unsigned int count = g.tile_cnt[tile], end = g.tile_end[tile];
+      s_key[threadIdx.x] = kEmptyKey;
+      __syncthreads();
+      const f4* pv = a.proj + (size_t)view * a.N;
+      auto walk = [&](int f, int sub, int step) {
+        TriRec t;
+        if (setup_tri(pv[a.faces[3 * f]], pv[a.faces[3 * f + 1]], pv[a.faces[3 * f + 2]], f, a.W, a.H, t))
+          raster_tri_in_tile(t, tx0, ty0, sub, step, s_key);
+      };
+      if (end <= g.capacity) {
+        int lg = 0;
+        while (lg < 3 && (count << (lg + 1)) <= kTilePix) ++lg;
+        const int sub = threadIdx.x & ((1 << lg) - 1);
+        for (unsigned int k = end - count + (threadIdx.x >> lg); k < end; k += kTilePix >> lg)
+          walk((int)g.bins[k], sub, 1 << lg);
+      } else {
+        for (int f = threadIdx.x; f < a.F; f += kTilePix) walk(f, 0, 1);
+      }
+      __syncthreads();
+      const int x = tx0 + (threadIdx.x % kTileW), y = ty0 + (threadIdx.x / kTileW);
+      // (the next tile clears this lane's own word)
+      if (x < a.W && y < a.H) resolve_pixel(a, view / a.C, view, x, y, s_key[threadIdx.x]);
+    }
+    if (back)
+      for (int y = by; y < min(by + kTileH, a.H); ++y) resolve_pixel(a, 0, bview, bx, y, kEmptyKey);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -548,11 +708,10 @@ size_t render_ws_fixed(const dcx_topo* t, const dcx_raster_cfg* c, int B, WsLayo
     const int tx = (c->width + kTileW - 1) / kTileW, ty = (c->height + kTileH - 1) / kTileH;
     const long long T = views * tx * ty;
     l.tiles = T;
-    l.tri = o; o = align256(o + sizeof(TriRec) * (size_t)views * F);
-    l.tile_cnt = o; o = align256(o + sizeof(unsigned int) * T);
-    l.tile_off = o; o = align256(o + sizeof(unsigned int) * (T + 1));
-    l.tile_fill = o; o = align256(o + sizeof(unsigned int) * T);
-    l.aux = o; o = align256(o + sizeof(unsigned int) * ((T + 1023) / 1024 + 1));
+    l.range = o; o = align256(o + sizeof(uint2) * (size_t)views * F);
+    l.tile_cnt = o; o = align256(o + sizeof(unsigned int) * (T + 2));
+    l.tile_end = o; o = align256(o + sizeof(unsigned int) * T);
+    l.full = o; o = align256(o + sizeof(unsigned int) * T);
     l.bins = o;
   }
   if (L) *L = l;
@@ -642,26 +801,24 @@ dcx_status render_fwd(const dcx_topo* t, const dcx_raster_cfg* c, int B, const f
   g.views = B * C;
   g.tiles_x = (c->width + kTileW - 1) / kTileW;
   g.tiles_per_view = g.tiles_x * ((c->height + kTileH - 1) / kTileH);
-  g.tri = (TriRec*)(w + L.tri);
+  g.tiles = L.tiles;
+  g.range = (uint2*)(w + L.range);
   g.tile_cnt = (unsigned int*)(w + L.tile_cnt);
-  g.tile_off = (unsigned int*)(w + L.tile_off);
-  g.tile_fill = (unsigned int*)(w + L.tile_fill);
+  g.tile_end = (unsigned int*)(w + L.tile_end);
+  g.full = (unsigned int*)(w + L.full);
   g.bins = (unsigned int*)(w + L.bins);
   g.capacity = (unsigned int)((ws_bytes - L.bins) / sizeof(unsigned int));
   const long long views = g.views;
-  hipLaunchKernelGGL(clear_u32_kernel, dim3(ceil_div(L.tiles, kB)), dim3(kB), 0, s, g.tile_cnt, L.tiles);
-  hipLaunchKernelGGL(clear_u32_kernel, dim3(ceil_div(L.tiles, kB)), dim3(kB), 0, s, g.tile_fill, L.tiles);
-  hipLaunchKernelGGL(project_kernel, dim3(ceil_div(views * N, kB)), dim3(kB), 0, s, vpos, ext, intr, N, C,
-                     (int)views, a.proj);
-  hipLaunchKernelGGL(face_normal_kernel, dim3(ceil_div((long long)B * F, kB)), dim3(kB), 0, s, vpos, t->faces,
-                     N, F, B, fnrm);
-  hipLaunchKernelGGL(vertex_normal_kernel, dim3(ceil_div((long long)B * N, kB)), dim3(kB), 0, s, fnrm,
-                     t->vf_off, t->vf_list, N, F, B, C, a.vnrm, vnormal);
-  hipLaunchKernelGGL(tri_setup_count_kernel, dim3(ceil_div(views * F, kB)), dim3(kB), 0, s, a, g);
-  st = exclusive_scan(g.tile_cnt, g.tile_off, (unsigned int*)(w + L.aux), L.tiles, s);
-  if (st) return st;
+  DCX_REQUIRE(L.tiles <= 4096ll * 1024, "dcx_render_fwd: %lld tiles exceed 4M", L.tiles);
+  const unsigned project_blocks = ceil_div(views * N, kB), normal_blocks = ceil_div((long long)B * N, kB);
+  hipLaunchKernelGGL(bin_prepare_kernel, dim3(project_blocks + ceil_div((long long)B * F, kB)), dim3(kB), 0, s, a, g,
+                     project_blocks, B, fnrm);
+  hipLaunchKernelGGL(bin_count_kernel, dim3(normal_blocks + ceil_div(views * F, kB)), dim3(kB), 0, s, a, g,
+                     normal_blocks, B, fnrm, t->vf_off, t->vf_list, (float*)(w + L.vnrm), vnormal);
+  hipLaunchKernelGGL(bin_offset_kernel, dim3(ceil_div(L.tiles, 4 * kB)), dim3(kB), 0, s, g);
   hipLaunchKernelGGL(bin_scatter_kernel, dim3(ceil_div(views * F, kB)), dim3(kB), 0, s, a, g);
-  hipLaunchKernelGGL(fine_raster_kernel, dim3((unsigned)L.tiles), dim3(kTilePix), 0, s, a, g);
+  hipLaunchKernelGGL(fine_raster_kernel, dim3((unsigned)(L.tiles < kFineBlocks ? L.tiles : kFineBlocks)),
+                     dim3(kTilePix), 0, s, a, g);
   return check_launch("dcx_render_fwd(binned)");
 }
 
@@ -742,8 +899,12 @@ extern "C" dcx_status dcx_render_fwd_noalloc(const dcx_topo* topo, const dcx_ras
   // the binned path needs at least kMinNoAllocBins tile-list entries beyond
   // the fixed part (fewer would only send more tiles down the overflow path)
   constexpr size_t kMinNoAllocBins = 65536;
+  // the batches that the array is documented to take: 48 bytes a (view, face),
+  // 8 of which hold its tile range and the rest more tile-list entries
   const size_t fixed = render_ws_fixed(topo, cfg, B, nullptr) +
-                       (plain_layout(cfg) ? 0 : sizeof(unsigned int) * kMinNoAllocBins);
+                       (plain_layout(cfg) ? 0
+                                          : (size_t)40 * B * cfg->num_cameras * topo->F +
+                                                sizeof(unsigned int) * kMinNoAllocBins);
   DCX_REQUIRE(fixed <= (size_t)DCX_RENDER_NOALLOC_SCRATCH_BYTES,
               "dcx_render_fwd_noalloc: this batch needs %zu bytes of scratch, more than the %zu of the static "
               "array (use dcx_render_fwd with a workspace)",

@@ -43,15 +43,16 @@ struct RenderArgs {
 struct BinArgs {
   int views, tiles_x, tiles_per_view;
   unsigned int capacity;
-  TriRec* tri;
-  unsigned int* tile_cnt;
-  unsigned int* tile_off;     // [tiles+1]
-  unsigned int* tile_fill;
-  unsigned int* bins;
+  long long tiles;            // views * tiles_per_view
+  uint2* range;               // [views, F] first and last tile of a face (x | y << 16)
+  unsigned int* tile_cnt;     // [tiles] list lengths, then their total and the number of tiles with a list
+  unsigned int* tile_end;     // [tiles] list cursors: start, after the scatter end
+  unsigned int* full;         // [tiles] the tiles with a list
+  unsigned int* bins;         // face ids
 };
 
 struct WsLayout {
-  size_t proj, fnrm, vnrm, keys, refcam, tri, tile_cnt, tile_off, tile_fill, aux, bins;
+  size_t proj, fnrm, vnrm, keys, refcam, range, tile_cnt, tile_end, full, bins;
   long long tiles;
 };
 

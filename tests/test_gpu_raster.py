@@ -204,3 +204,38 @@ def test_cuda_renderer_gpu_wrapper_and_gradient_wiring():
                                   extrinsics_input=ext, intrinsics_input=intr)
     r2.getRenderBufferTF().sum().backward()
     assert torch.count_nonzero(vp2.grad) == 0
+
+
+@pytest.mark.parametrize("W,H,order", [(200, 90, "mixed"), (1100, 40, "mixed"), (65, 700, "shuffled"), (300, 300, "fan")])
+def test_binning_of_small_large_and_scattered_triangles(W, H, order):
+    """Bit-exact against the oracle: triangles of a pixel, around 64 pixels
+    wide (where the walk changes to 64 bits), over more than 16 tiles and over
+    the whole image, in one wavefront; faces without any order; a vertex with
+    300 faces."""
+    rng = np.random.default_rng(W)
+    ext = np.array([[1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0]], np.float32)
+    intr = np.array([[1, 0, 0, 0, 1, 0, 0, 0, 1]], np.float32)  # (x z, y z, z) is seen at (x, y)
+    if order == "fan":
+        a = np.linspace(0, 2 * np.pi, 301)[:-1]
+        xy = np.concatenate([[[150.2, 149.7]], np.stack([150 + 140 * np.cos(a), 150 + 140 * np.sin(a)], 1)])
+        z = np.concatenate([[1.0], rng.uniform(1, 2, 300)])
+        i = np.arange(300)
+        faces = np.stack([0 * i, 1 + i, 1 + (i + 1) % 300], 1).astype(np.int32)
+    else:
+        sizes = np.concatenate([rng.uniform(0.3, 3, 400), rng.choice([31.9, 32.0, 32.1], 60), rng.uniform(60, 200, 20), [2000.0]])
+        xy = np.concatenate([rng.uniform(0, [W, H]) + s * rng.uniform(-1, 1, (3, 2)) for s in sizes])
+        # corners exactly 64 pixels (and one 256th more) apart
+        xy[-63:-60] = np.array([[8.5, 4.5], [72.5, 4.5], [8.5, 30.5]])
+        xy[-66:-63] = np.array([[8.5, 4.5], [72.5 + 1 / 256, 4.5], [8.5, 30.5]])
+        z = rng.uniform(1, 5, len(xy))
+        faces = np.arange(len(xy), dtype=np.int32).reshape(-1, 3)
+        faces = rng.permutation(faces, axis=0) if order == "shuffled" else faces
+    V = np.concatenate([xy * z[:, None], z[:, None]], 1)[None].astype(np.float32)
+    col = rng.uniform(0, 1, V.shape).astype(np.float32)
+    topo = renderer.Topology(faces, V.shape[1])
+    cfg = renderer.make_cfg(1, W, H)
+    bary, face, render, vn = renderer.render_forward(topo, cfg, _t(V), _t(col), None, None, _t(ext), _t(intr))
+    of, ob, orr, ovn = orc.raster_fwd(faces, V, ext, intr, H, W, vcol=col)
+    for got, ref in ((face, of), (bary, ob), (render, orr), (vn, ovn)):
+        assert np.array_equal(got.cpu().numpy().reshape(np.shape(ref)), ref)
+    assert (of >= 0).mean() > 0.3
