@@ -99,8 +99,9 @@ __global__ __launch_bounds__(kB) void face_normal_kernel(const float* __restrict
 // vertex's loads are issued eight at a time; the few vertices with more than
 // kManyFaces faces (the poles of a mesh: a hundred and more) are loaded by the
 // whole wavefront and added up in the same order, since a lane that walks such
-// a list load by load is the last of the launch (24 us of 24 for 50k vertices
-// and 8 views; MEASUREDVN).  All lanes of a wavefront call it.
+// a list load by load is the last of the launch (24 us for 50k vertices and 8
+// views; with the tile counts in the same launch 24 now).  All lanes of a
+// wavefront call it.
 constexpr int kManyFaces = 16;
 __device__ __forceinline__ void vertex_normal_one(const float* __restrict__ fn, const int* __restrict__ off,
                                                   const int* __restrict__ lst, int N, int F, int B, int C,

@@ -1,22 +1,29 @@
 // Rasterizer backward (CudaRendererGradGpu) on gfx950.
 //
-// One lane per pixel, pixels in row-major order so a wavefront covers 64
-// consecutive pixels of a row.  Each covered pixel recomputes its
-// barycentric Jacobian from the stored face id (nothing per-pixel is kept
-// from the forward pass besides the reference's face / barycentric buffers),
-// forms its 9 position and 9 colour contributions, and the wavefront
-// combines runs of equal face ids with a segmented shuffle scan: only the
-// last lane of each run issues the 18 global atomics.  SH gradients (27
-// floats per camera, hit by every pixel of that camera) are reduced per
-// block in LDS first.
+// Gather form (with the workspace that dcx_render_bwd_workspace_size asks for):
+// four lanes per (view, face) find the pixels of the face's box whose stored
+// face id is its own, form their contributions from the stored barycentrics
+// (nothing per-pixel is kept from the forward pass besides the reference's
+// face / barycentric buffers) and sum them in registers; eight lanes per
+// vertex then add up the records of its faces in all views.  No atomics but
+// the texture's and one flush of the SH gradients a workgroup, and the sums
+// have a fixed order.
+//
+// Scatter form (the remaining pixels: faces over more than kGatherBox pixels,
+// face buffers that were not rendered from these positions; and everything,
+// for callers without that workspace): one lane per pixel, pixels in row-major
+// order so a wavefront covers 64 consecutive pixels of a row; the wavefront
+// combines runs of equal face ids with a segmented shuffle scan and only the
+// last lane of each run issues the global atomics.  SH gradients (27 floats
+// per camera, hit by every pixel of that camera) are reduced per block in LDS
+// first.
 //
 // Shaded mode also differentiates the vertex normals (sums of the adjacent
-// unnormalised face normals, CUDABasedRasterizationGrad.cu:441-493): the
-// pixel kernel reduces dL/d(vertex normal) per vertex into a [B,N,3]
-// workspace (9 more floats in the same segmented scan), then one lane per
-// vertex walks its faces and applies the face-normal Jacobians
-// (RendererUtil.h:492-540) -- a deterministic gather in place of the
-// reference's per-pixel loop over the faces around each corner.
+// unnormalised face normals, CUDABasedRasterizationGrad.cu:441-493): both
+// forms sum dL/d(vertex normal) per vertex into a [B,N,3] workspace, then the
+// vertices' faces apply the face-normal Jacobians (RendererUtil.h:492-540) --
+// a deterministic gather in place of the reference's per-pixel loop over the
+// faces around each corner.
 #include "raster_common.hpp"
 #include "raster_internal.hpp"
 
@@ -46,28 +53,90 @@ struct BwdArgs {
   float* g_tex;
   float* g_sh;
   float* g_vn;            // [B,N,3] shaded only
+  // gather form
+  float* rec;             // [B,C,F,rec_n] sums of a face's pixels in a view: position, colour, normal of 3 corners
+  uint2* box;             // [B,C,F] a face's box: x0 | y0 << 16, nx | ny << 10 | (record written) << 20
+  unsigned int* rest_n;   // pixel groups left to the scatter form, and
+  unsigned int* rest;     // which ([pixels / kB] at most)
+  int rec_n, rec_col, rec_vn;
 };
 
+// Faces whose box holds more pixels are left to the scatter form, where a
+// large triangle's pixels are spread over many wavefronts and its long runs
+// combine well (a wavefront of the gather that held only such faces, the caps
+// of a limb, took 4 ms).
+constexpr int kGatherBox = 256;
+constexpr int kFaceLanes = 4;
+
+// Pixels that a face can cover: centres in the bounding box of its projection
+// (and of its corners snapped to 1/256 pixel).  nx = 0: none, or not gathered.
+struct FaceBox {
+  int x0, y0, nx, ny;
+  __device__ __forceinline__ bool has(int x, int y) const {
+    return x >= x0 && x < x0 + nx && y >= y0 && y < y0 + ny;
+  }
+};
+__device__ __forceinline__ FaceBox face_box(f4 p0, f4 p1, f4 p2, int W, int H) {
+  FaceBox b{0, 0, 0, 0};
+  if (!(p0.w > 0.f && p1.w > 0.f && p2.w > 0.f)) return b;
+  constexpr float kMargin = 1.f / 256.f;
+  const float x0 = fmaxf(ceilf(fminf(p0.x, fminf(p1.x, p2.x)) - 0.5f - kMargin), 0.f);
+  const float y0 = fmaxf(ceilf(fminf(p0.y, fminf(p1.y, p2.y)) - 0.5f - kMargin), 0.f);
+  const float x1 = fminf(floorf(fmaxf(p0.x, fmaxf(p1.x, p2.x)) - 0.5f + kMargin), (float)(W - 1));
+  const float y1 = fminf(floorf(fmaxf(p0.y, fmaxf(p1.y, p2.y)) - 0.5f + kMargin), (float)(H - 1));
+  if (!(x0 <= x1 && y0 <= y1 && (x1 - x0 + 1.f) * (y1 - y0 + 1.f) <= (float)kGatherBox)) return b;
+  b.x0 = (int)x0; b.y0 = (int)y0; b.nx = (int)x1 - b.x0 + 1; b.ny = (int)y1 - b.y0 + 1;
+  return b;
+}
+__device__ __forceinline__ FaceBox unpack_box(uint2 w) {
+  return {(int)(w.x & 0xffff), (int)(w.x >> 16), (int)(w.y & 0x3ff), (int)((w.y >> 10) & 0x3ff)};
+}
+
 // imageGradient of RendererUtil.h:566-620 at a (possibly fractional) point:
-// the sample index is formed as (int)((y + yy) * W + (x + xx)) in float.
-__device__ void image_gradient(const float* img, float x, float y, int W, int H, int fs, f3& du, f3& dv) {
+// the sample index is formed as (int)((y + yy) * W + (x + xx)) in float.  kFs:
+// the filter size where it is known, so that a row's loads are issued
+// together (one tap after the other, a 5 x 5 filter was the longest part of a
+// pixel); 0: any.
+template <int kFs>
+__device__ __forceinline__ void image_gradient_of(const float* img, float x, float y, int W, int H, int fs_, f3& du,
+                                                  f3& dv) {
+  const int fs = kFs ? kFs : fs_;
   du = mk3(0.f, 0.f, 0.f);
   dv = mk3(0.f, 0.f, 0.f);
   if (!(x >= (float)(fs + 1) && y >= (float)(fs + 1) && x < (float)(W - (fs + 1)) && y < (float)(H - (fs + 1))))
     return;
   float norm = 0.f;
-  for (int yy = -fs; yy <= fs; ++yy)
-    for (int xx = -fs; xx <= fs; ++xx) {
-      const f3 I = ld3(img + (size_t)(int)((y + (float)yy) * (float)W + (x + (float)xx)) * 3);
-      const float den = (float)(xx * xx + yy * yy);
-      float gu = 0.f, gv = 0.f;
-      if (den != 0.f) { gu = (float)xx / den; gv = (float)yy / den; }
-      du = du + I * gu;
-      dv = dv + I * gv;
-      norm += fabsf(gu);
+  auto tap = [&](int xx, int yy, f3 I) {
+    const float den = (float)(xx * xx + yy * yy);
+    float gu = 0.f, gv = 0.f;
+    if (den != 0.f) { gu = (float)xx / den; gv = (float)yy / den; }
+    du = du + I * gu;
+    dv = dv + I * gv;
+    norm += fabsf(gu);
+  };
+  auto at = [&](int xx, int yy) {
+    return ld3(img + (size_t)(int)((y + (float)yy) * (float)W + (x + (float)xx)) * 3);
+  };
+  if (kFs) {
+#pragma unroll
+    for (int yy = -kFs; yy <= kFs; ++yy) {
+      f3 I[2 * kFs + 1];
+#pragma unroll
+      for (int xx = -kFs; xx <= kFs; ++xx) I[xx + kFs] = at(xx, yy);
+#pragma unroll
+      for (int xx = -kFs; xx <= kFs; ++xx) tap(xx, yy, I[xx + kFs]);
     }
+  } else {
+    for (int yy = -fs; yy <= fs; ++yy)
+      for (int xx = -fs; xx <= fs; ++xx) tap(xx, yy, at(xx, yy));
+  }
   du = mk3(du.x / norm, du.y / norm, du.z / norm);
   dv = mk3(dv.x / norm, dv.y / norm, dv.z / norm);
+}
+__device__ __forceinline__ void image_gradient(const float* img, float x, float y, int W, int H, int fs, f3& du, f3& dv) {
+  if (fs == 1) image_gradient_of<1>(img, x, y, W, H, fs, du, dv);
+  else if (fs == 2) image_gradient_of<2>(img, x, y, W, H, fs, du, dv);
+  else image_gradient_of<0>(img, x, y, W, H, fs, du, dv);
 }
 
 // d(b0, b1, 1-b0-b1)/d(world vertex positions) contracted with gb = dL/d weights.
@@ -146,19 +215,27 @@ __device__ __forceinline__ bool seg_reduce(float* v, int key, int key2) {
   return lane == 63 || next != key || next2 != key2;
 }
 
-__global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
+template <bool kRest>
+__device__ __forceinline__ void bwd_group(const BwdArgs& a, unsigned int group) {
   __shared__ float s_sh[27];
   const long long HW = (long long)a.H * a.W;
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
+  const long long i = (long long)group * kB + threadIdx.x;
   const bool valid = i < (long long)a.B * a.C * HW;
   const int view = valid ? (int)(i / HW) : 0;
   // SH accumulation is per camera; a block never straddles two views when HW % 256 == 0,
   // otherwise the per-lane atomics below handle the rest.
-  const int view0 = (int)(((long long)blockIdx.x * kB) / HW);
-  const bool block_one_view = ((long long)blockIdx.x * kB + kB - 1) / HW == view0;
-  if (a.shaded && a.g_sh && threadIdx.x < 27) s_sh[threadIdx.x] = 0.f;
-  if (a.shaded && a.g_sh) __syncthreads();
-  const int f = valid ? a.face[i] : -1;
+  const int view0 = (int)(((long long)group * kB) / HW);
+  const bool block_one_view = ((long long)group * kB + kB - 1) / HW == view0;
+  if (a.shaded && a.g_sh) {
+    __syncthreads();  // the group before
+    if (threadIdx.x < 27) s_sh[threadIdx.x] = 0.f;
+    __syncthreads();
+  }
+  int f = valid ? a.face[i] : -1;
+  if (kRest && f >= 0) {
+    const int p = (int)(i - (long long)view * HW);
+    if (unpack_box(a.box[(size_t)view * a.F + f]).has(p % a.W, p / a.W)) f = -1;
+  }
   float acc[27];  // 0-8 position, 9-17 colour, 18-26 vertex-normal gradients of the 3 corners
 #pragma unroll
   for (int k = 0; k < 27; ++k) acc[k] = 0.f;
@@ -300,7 +377,9 @@ __global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
     for (int k = 0; k < 3; ++k) { acc[3 * k] = gx[k].x; acc[3 * k + 1] = gx[k].y; acc[3 * k + 2] = gx[k].z; }
   }
   // Combine runs of equal (view, face) within the wavefront.
-  const bool tail = a.shaded ? seg_reduce<27>(acc, f, view) : seg_reduce<18>(acc, f, view);
+  // (a wavefront without a covered pixel has nothing to combine)
+  bool tail = false;
+  if (__ballot(f >= 0)) tail = a.shaded ? seg_reduce<27>(acc, f, view) : seg_reduce<18>(acc, f, view);
   if (f >= 0 && tail) {
     float* gp = a.g_vpos + (size_t)b * a.N * 3;
     const int idx[3] = {i0, i1, i2};
@@ -331,7 +410,7 @@ __global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
   }
   if (a.shaded && a.g_sh) {
     if (block_one_view) {
-      for (int k = 0; k < 27; ++k) {
+      for (int k = 0; k < 27 && __ballot(have_sh); ++k) {
         const float t = wave_sum(have_sh ? shv[k] : 0.f);
         if ((threadIdx.x & 63) == 0 && t != 0.f) atomicAdd(&s_sh[k], t);
       }
@@ -344,35 +423,473 @@ __global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
   }
 }
 
-// One lane per (mesh, vertex): n_v = sum over the faces around v (one entry
-// per corner) of N_f = (v1 - v0) x (v2 - v0).  With G_f = sum of dL/dn over
-// the three corners of f, dL/dv0 = (e1 - e2) x G_f, dL/dv1 = e2 x G_f,
-// dL/dv2 = G_f x e1 (e1 = v1 - v0, e2 = v2 - v0); v takes the terms of the
-// corners it occupies, once per face (a face listing v twice appears twice,
-// consecutively, in v's list).
+// kRest: only the pixels that the gather form did not take, a.rest's groups of
+// kB pixels in turn; otherwise the workgroup's own group.
+template <bool kRest>
+__global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
+  if (kRest) {
+    const unsigned int n = *a.rest_n;
+    for (unsigned int q = blockIdx.x; q < n; q += gridDim.x) bwd_group<true>(a, a.rest[q]);
+  } else {
+    bwd_group<false>(a, blockIdx.x);
+  }
+}
+
+// Sums of one face's pixels in one view.
+template <bool kTex, bool kShaded>
+struct FaceSums {
+  float gu[3], gv[3], giz[3];  // dL/d(image position, 1/z) of the corners through the barycentrics
+  f3 gx[3];                    // dL/d(world position) through the target's gradient
+  f3 gc[kTex ? 1 : 3];         // dL/d(vertex colour)
+  f3 gn[kShaded ? 3 : 1];      // dL/d(vertex normal)
+  float sh[kShaded ? 27 : 1];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) { gu[i] = gv[i] = giz[i] = 0.f; gx[i] = mk3(0.f, 0.f, 0.f); }
+#pragma unroll
+    for (int i = 0; i < (kTex ? 1 : 3); ++i) gc[i] = mk3(0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < (kShaded ? 3 : 1); ++i) gn[i] = mk3(0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < (kShaded ? 27 : 1); ++i) sh[i] = 0.f;
+  }
+};
+
+// What a face's pixels share.
+template <bool kTex, bool kShaded>
+struct FaceInfo {
+  f3 X[3], vn[kTex || kShaded ? 3 : 1], col[kTex ? 1 : 3];
+  f4 p[3];
+  float t6[kTex ? 6 : 1];
+  FaceBox box;
+  __device__ __forceinline__ void load(const BwdArgs& a, int view, int b, int f) {
+    const float* E = a.ext + (size_t)view * 12;
+    const float* K = a.intr + (size_t)view * 9;
+    const float* vp = a.vpos + (size_t)b * a.N * 3;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int v = a.faces[3 * f + k];
+      X[k] = ld3(vp + 3 * v);
+      p[k] = project_vertex(E, K, vp + 3 * v);
+      if (kTex || kShaded) vn[k] = ld3(a.vnormal + ((size_t)view * a.N + v) * 3);
+      if (!kTex) col[k] = ld3(a.vcol + ((size_t)b * a.N + v) * 3);
+    }
+    if (kTex)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) t6[k] = a.tc[(size_t)f * 6 + k];
+    box = face_box(p[0], p[1], p[2], a.W, a.H);
+  }
+};
+
+// Adds pixel (x, y) of the face to its sums; the same terms as in
+// render_bwd_kernel, with what is linear in the pixels left to face_record.
+template <bool kTex, bool kShaded>
+__device__ __forceinline__ void add_pixel(const BwdArgs& a, int view, int b, const FaceInfo<kTex, kShaded>& I, int x,
+                                          int y, FaceSums<kTex, kShaded>& S) {
+  const long long HW = (long long)a.H * a.W, i = (long long)view * HW + (long long)y * a.W + x;
+  const float px = (float)x + 0.5f, py = (float)y + 0.5f;
+  const float* E = a.ext + (size_t)view * 12;
+  const float* K = a.intr + (size_t)view * 9;
+  const float wa = a.bary[2 * i], wb = a.bary[2 * i + 1];
+  const float w[3] = {wa, wb, 1.f - wa - wb};
+  const f3 g = ld3(a.g_render + 3 * i);
+  f3 n = mk3(0.f, 0.f, 0.f), pn = n;
+  float pl = 1.f;
+  bool flipped = false;
+  const float* shc = kShaded ? a.sh + (size_t)view * 27 : nullptr;
+  if (kTex || kShaded) {
+    pn = mk3(w[0] * I.vn[0].x + w[1] * I.vn[1].x + w[2] * I.vn[2].x, w[0] * I.vn[0].y + w[1] * I.vn[1].y + w[2] * I.vn[2].y,
+             w[0] * I.vn[0].z + w[1] * I.vn[1].z + w[2] * I.vn[2].z);
+    pl = sqrtf(dot(pn, pn));
+    n = mk3(pn.x / pl, pn.y / pl, pn.z / pl);
+    if (dot(n, world_ray_dir(E, K, px, py)) > 0.f) { n = -n; flipped = true; }
+  }
+  f3 light = mk3(1.f, 1.f, 1.f);
+  if (kShaded) light = sh_shade(mk3(1.f, 1.f, 1.f), n, shc);
+  const f3 ga = mk3(g.x * light.x, g.y * light.y, g.z * light.z);
+  f3 alb = mk3(0.f, 0.f, 0.f);
+  float gw[3];
+  if (!kTex) {
+    alb = I.col[0] * w[0] + I.col[1] * w[1] + I.col[2] * w[2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      S.gc[k] = S.gc[k] + ga * w[k];
+      gw[k] = dot(ga, I.col[k]);
+    }
+  } else {
+    float U0 = (I.t6[0] * w[0] + I.t6[2] * w[1] + I.t6[4] * w[2]) * (float)a.TW;
+    float V0 = ((1.f - I.t6[1]) * w[0] + (1.f - I.t6[3]) * w[1] + (1.f - I.t6[5]) * w[2]) * (float)a.TH;
+    U0 = fminf(fmaxf(U0, 0.f), (float)(a.TW - 1));
+    V0 = fminf(fmaxf(V0, 0.f), (float)(a.TH - 1));
+    const float* tx = a.tex + (size_t)b * a.TH * a.TW * 3;
+    if (kShaded) {
+      const float LU = (float)(int)(U0 - 0.5f) + 0.5f, HU = LU + 1.f;
+      const float LV = (float)(int)(V0 - 0.5f) + 0.5f, HV = LV + 1.f;
+      auto at = [&](float uu, float vv) { return ld3(tx + ((size_t)(int)vv * a.TW + (int)uu) * 3); };
+      alb = (at(LU, LV) * (U0 - LU) + at(HU, LV) * (HU - U0)) * (V0 - LV) +
+            (at(LU, HV) * (U0 - LU) + at(HU, HV) * (HU - U0)) * (HV - V0);
+    }
+    if (!flipped && a.g_tex) {
+      float* gt = a.g_tex + (size_t)b * a.TH * a.TW * 3 + ((size_t)(int)(V0 - 0.5f) * a.TW + (int)(U0 - 0.5f)) * 3;
+      atomicAdd(gt, ga.x); atomicAdd(gt + 1, ga.y); atomicAdd(gt + 2, ga.z);
+    }
+    f3 du, dv;
+    image_gradient(tx, U0, V0, a.TW, a.TH, a.tex_fs, du, dv);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float su = I.t6[2 * k] * (float)a.TW, sv = (1.f - I.t6[2 * k + 1]) * (float)a.TH;
+      gw[k] = ga.x * (du.x * su + dv.x * sv) + ga.y * (du.y * su + dv.y * sv) + ga.z * (du.z * su + dv.z * sv);
+    }
+  }
+  if (kShaded) {
+    const float basis[9] = {1.f, n.y, n.z, n.x, n.x * n.y, n.z * n.y, 3.f * n.z * n.z - 1.f, n.x * n.z, n.x * n.x - n.y * n.y};
+    const float gc[3] = {g.x * alb.x, g.y * alb.y, g.z * alb.z};
+    f3 gn = mk3(0.f, 0.f, 0.f);
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) S.sh[9 * ch + k] += gc[ch] * basis[k];
+      const float* s = shc + 9 * ch;
+      const f3 Jn = mk3(s[3] + s[4] * n.y + s[7] * n.z + s[8] * 2.f * n.x,
+                        s[1] + s[4] * n.x + s[5] * n.z + s[8] * -2.f * n.y,
+                        s[2] + s[5] * n.y + s[6] * 6.f * n.z + s[7] * n.x);
+      gn = gn + Jn * gc[ch];
+    }
+    const float sg = flipped ? -1.f : 1.f;
+    const f3 nn = mk3(pn.x / pl, pn.y / pl, pn.z / pl);
+    const float dg = sg * dot(gn, nn);
+    const f3 gun = mk3((sg * gn.x - nn.x * dg) / pl, (sg * gn.y - nn.y * dg) / pl, (sg * gn.z - nn.z * dg) / pl);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      gw[k] += dot(gun, I.vn[k]);
+      S.gn[k] = S.gn[k] + gun * w[k];
+    }
+  }
+  // through the barycentrics to the corners' image positions and 1/z (bary_vjp)
+  float e[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const f4 pj = I.p[k == 2 ? 0 : k + 1], pk = I.p[k == 0 ? 2 : k - 1];
+    e[k] = (pk.x - pj.x) * (py - pj.y) - (pk.y - pj.y) * (px - pj.x);
+  }
+  const float q0 = e[0] * I.p[0].w, q1 = e[1] * I.p[1].w, q2 = e[2] * I.p[2].w;
+  const float Q = q0 + q1 + q2;
+  const float b0 = q0 / Q, b1 = q1 / Q;
+  const float g0 = gw[0] - gw[2], g1 = gw[1] - gw[2];
+  const float s = g0 * b0 + g1 * b1;
+  const float gq[3] = {(g0 - s) / Q, (g1 - s) / Q, (0.f - s) / Q};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int jj = k == 2 ? 0 : k + 1, kk = k == 0 ? 2 : k - 1;
+    const f4 pj = I.p[jj], pk = I.p[kk];
+    S.giz[k] += gq[k] * e[k];
+    const float ge = gq[k] * I.p[k].w;
+    S.gu[jj] += ge * (pk.y - py);
+    S.gv[jj] += ge * (px - pk.x);
+    S.gu[kk] += ge * (py - pj.y);
+    S.gv[kk] += ge * (pj.x - px);
+  }
+  if (a.target) {
+    f3 du, dv;
+    image_gradient(a.target + (size_t)view * HW * 3, (float)x, (float)y, a.W, a.H, a.img_fs, du, dv);
+    const float gu = -dot(g, du), gvv = -dot(g, dv);
+    const f3 fp = I.X[0] * w[0] + I.X[1] * w[1] + I.X[2] * w[2];
+    const float xc = E[0] * fp.x + E[1] * fp.y + E[2] * fp.z + E[3];
+    const float yc = E[4] * fp.x + E[5] * fp.y + E[6] * fp.z + E[7];
+    const float zc = E[8] * fp.x + E[9] * fp.y + E[10] * fp.z + E[11];
+    const float hx = K[0] * xc + K[1] * yc + K[2] * zc;
+    const float hy = K[3] * xc + K[4] * yc + K[5] * zc;
+    const float hz = K[6] * xc + K[7] * yc + K[8] * zc;
+    if (fabsf(hz) > 0.0001f) {
+      const float gh0 = gu / hz, gh1 = gvv / hz, gh2 = -(gu * hx + gvv * hy) / (hz * hz);
+      const float cx = K[0] * gh0 + K[3] * gh1 + K[6] * gh2;
+      const float cy = K[1] * gh0 + K[4] * gh1 + K[7] * gh2;
+      const float cz = K[2] * gh0 + K[5] * gh1 + K[8] * gh2;
+      const f3 gX = mk3(E[0] * cx + E[4] * cy + E[8] * cz, E[1] * cx + E[5] * cy + E[9] * cz,
+                        E[2] * cx + E[6] * cy + E[10] * cz);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) S.gx[k] = S.gx[k] + gX * w[k];
+    }
+  }
+}
+
+// The face's record: its corners' image-space sums taken to world space once.
+template <bool kTex, bool kShaded>
+__device__ __forceinline__ void face_record(const BwdArgs& a, int view, const FaceInfo<kTex, kShaded>& I,
+                                            const FaceSums<kTex, kShaded>& S, float* r) {
+  const float* E = a.ext + (size_t)view * 12;
+  const float* K = a.intr + (size_t)view * 9;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const f4 p = I.p[i];
+    const float gh0 = S.gu[i] / p.z, gh1 = S.gv[i] / p.z;
+    const float gh2 = -(S.gu[i] * p.x + S.gv[i] * p.y) / p.z - S.giz[i] * p.w * p.w;
+    const float gx = K[0] * gh0 + K[3] * gh1 + K[6] * gh2;
+    const float gy = K[1] * gh0 + K[4] * gh1 + K[7] * gh2;
+    const float gz = K[2] * gh0 + K[5] * gh1 + K[8] * gh2;
+    r[3 * i] = E[0] * gx + E[4] * gy + E[8] * gz + S.gx[i].x;
+    r[3 * i + 1] = E[1] * gx + E[5] * gy + E[9] * gz + S.gx[i].y;
+    r[3 * i + 2] = E[2] * gx + E[6] * gy + E[10] * gz + S.gx[i].z;
+    if (!kTex && a.rec_col) {
+      float* c = r + a.rec_col + 3 * i;
+      c[0] = S.gc[i].x; c[1] = S.gc[i].y; c[2] = S.gc[i].z;
+    }
+    if (kShaded) {
+      float* c = r + a.rec_vn + 3 * i;
+      c[0] = S.gn[i].x; c[1] = S.gn[i].y; c[2] = S.gn[i].z;
+    }
+  }
+}
+
+// Sums of every member but the SH gradients over a face's lanes, in all of them.
+template <bool kTex, bool kShaded>
+__device__ __forceinline__ void lanes_total(FaceSums<kTex, kShaded>& S) {
+  static_assert(kFaceLanes == 4, "a quad");
+  auto sum4 = [](float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));  // 1 apart
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));  // 2 apart
+    return v;
+  };
+  auto f3sum = [&](f3 v) { return mk3(sum4(v.x), sum4(v.y), sum4(v.z)); };
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    S.gu[i] = sum4(S.gu[i]); S.gv[i] = sum4(S.gv[i]); S.giz[i] = sum4(S.giz[i]);
+    S.gx[i] = f3sum(S.gx[i]);
+    if (!kTex) S.gc[i] = f3sum(S.gc[i]);
+    if (kShaded) S.gn[i] = f3sum(S.gn[i]);
+  }
+}
+
+// kFaceLanes lanes per face, one view per workgroup row.  The box is searched
+// first (its face ids, four loads at a time, into a bit a pixel), so that the
+// wavefront runs the long part of the code as often as its lane with the most
+// pixels of its own, not as often as the largest box.
+// Pixel-parallel with segmented scans and up to 27 atomics a run, this part
+// took 570 us for 25k vertices, 4 views of 1024 x 1024, shaded vertex colours
+// (903 us textured, 50k vertices, 8 views of 1285 x 940); now 187 here, 29 in
+// the vertex gather and 97 for the pixels left over (413, 61 and 140).  What
+// bounds it is the latency of a pixel's loads at two wavefronts a SIMD: the
+// sums of a shaded face are 63 registers.
+template <bool kTex, bool kShaded>
+__global__ __launch_bounds__(kB) void face_gather_kernel(BwdArgs a) {
+  __shared__ float s_sh[32];
+  const int view = blockIdx.y, b = view / a.C, lane = threadIdx.x & 63, sub = threadIdx.x % kFaceLanes;
+  const int f = (blockIdx.x * kB + threadIdx.x) / kFaceLanes;
+  const bool in = f < a.F;
+  if (kShaded) {
+    if (threadIdx.x < 32) s_sh[threadIdx.x] = 0.f;
+    __syncthreads();
+  }
+  FaceInfo<kTex, kShaded> I;
+  I.load(a, view, b, in ? f : a.F - 1);
+  const int n = in ? I.box.nx * I.box.ny : 0;
+  // k / nx for k < kGatherBox: (k + 1/2) / nx is at least 1 / 512 away from a whole number
+  const float inv_nx = __builtin_amdgcn_rcpf((float)I.box.nx);
+  auto row_of = [&](int k) { return (int)(((float)k + 0.5f) * inv_nx); };
+  const int* ids = a.face + (size_t)view * a.H * a.W;
+  unsigned long long mine = 0;  // bit j: pixel sub + kFaceLanes * j
+  static_assert(kGatherBox <= 64 * kFaceLanes, "a bit a pixel");
+  for (int j0 = 0; j0 * kFaceLanes + sub < n; j0 += 4) {
+    int id[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k = min((j0 + j) * kFaceLanes + sub, n - 1), y = row_of(k);
+      id[j] = ids[(size_t)(I.box.y0 + y) * a.W + I.box.x0 + k - y * I.box.nx];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      mine |= (unsigned long long)(id[j] == f && (j0 + j) * kFaceLanes + sub < n) << (j0 + j);
+  }
+  FaceSums<kTex, kShaded> S;
+  S.clear();
+  const bool found = mine != 0;
+  while (mine) {
+    const int k = (__ffsll(mine) - 1) * kFaceLanes + sub, y = row_of(k);
+    mine &= mine - 1;
+    add_pixel<kTex, kShaded>(a, view, b, I, I.box.x0 + k - y * I.box.nx, I.box.y0 + y, S);
+  }
+  const size_t at = (size_t)view * a.F + f;
+  const unsigned long long hits = __ballot(found);
+  if (hits) {
+    lanes_total<kTex, kShaded>(S);
+    const bool any = ((hits >> (lane - sub)) & ((1u << kFaceLanes) - 1u)) != 0;
+    if (sub == 0 && any) face_record<kTex, kShaded>(a, view, I, S, a.rec + at * a.rec_n);
+    if (sub == 0 && in)
+      a.box[at] = make_uint2((unsigned)I.box.x0 | (unsigned)I.box.y0 << 16,
+                             (unsigned)I.box.nx | (unsigned)I.box.ny << 10 | (any ? 1u << 20 : 0u));
+  } else if (sub == 0 && in) {
+    a.box[at] = make_uint2((unsigned)I.box.x0 | (unsigned)I.box.y0 << 16, (unsigned)I.box.nx | (unsigned)I.box.ny << 10);
+  }
+  if (kShaded && a.g_sh) {
+    if (hits) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = 8 * r + k < 27 ? S.sh[8 * r + k < 27 ? 8 * r + k : 0] : 0.f;
+        const float t = wave_sum8(v);
+        if (lane < 8) atomicAdd(&s_sh[8 * r + lane], t);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 27 && s_sh[threadIdx.x] != 0.f)
+      atomicAdd(a.g_sh + (size_t)view * 27 + threadIdx.x, s_sh[threadIdx.x]);
+  }
+}
+
+constexpr int kVertexLanes = 8;
+constexpr int kManyFaces = 32;  // vertices with more faces are a whole wavefront's
+
+// Sum over a group of 8 lanes, in all of them.
+__device__ __forceinline__ float sum8(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));   // 1 apart
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));   // 2 apart
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));  // half mirror
+  return v;
+}
+
+// Calls add(face id) for the vertex's faces, each once (a face that lists the
+// vertex twice stands twice in its list, one after the other), and stores the
+// sums: eight lanes a vertex, or the wavefront for vertices with many faces
+// (the poles of a mesh; eight lanes walk 130 of them after the launch is done).
+template <int kNV, class Add, class Store>
+__device__ __forceinline__ void for_vertex_faces(const int* off, const int* lst, int N, int B, Add add, Store store) {
+  const long long i = ((long long)blockIdx.x * kB + threadIdx.x) / kVertexLanes;
+  const int sub = threadIdx.x % kVertexLanes, lane = threadIdx.x & 63;
+  const bool in = i < (long long)B * N;
+  const int b = in ? (int)(i / N) : 0, v = in ? (int)(i - (long long)b * N) : 0;
+  const int k0 = in ? off[v] : 0, k1 = in ? off[v + 1] : 0;
+  float s[kNV];
+#pragma unroll
+  for (int j = 0; j < kNV; ++j) s[j] = 0.f;
+  const bool many = k1 - k0 > kManyFaces;
+  if (!many)
+    for (int k = k0 + sub; k < k1; k += kVertexLanes) {
+      const int f = lst[k];
+      if (k == k0 || lst[k - 1] != f) add(b, v, f, s);
+    }
+#pragma unroll
+  for (int j = 0; j < kNV; ++j) s[j] = sum8(s[j]);
+  if (in && !many && sub == 0) store(i, s);
+  for (unsigned long long todo = __ballot(many && sub == 0); todo; todo &= todo - 1) {
+    const int src = __ffsll(todo) - 1;
+    const int c0 = __builtin_amdgcn_readlane(k0, src), c1 = __builtin_amdgcn_readlane(k1, src);
+    const int cb = __builtin_amdgcn_readlane(b, src), cv = __builtin_amdgcn_readlane(v, src);
+    float t[kNV];
+#pragma unroll
+    for (int j = 0; j < kNV; ++j) t[j] = 0.f;
+    for (int k = c0 + lane; k < c1; k += 64) {
+      const int f = lst[k];
+      if (k == c0 || lst[k - 1] != f) add(cb, cv, f, t);
+    }
+#pragma unroll
+    for (int j = 0; j < kNV; ++j) t[j] = wave_sum(t[j]);
+    if (lane == src) store(i, t);
+  }
+}
+
+// Pixels that no face's box took, four a lane: their groups into a.rest.
+__device__ __forceinline__ void find_rest(const BwdArgs& a, unsigned int block) {
+  __shared__ unsigned int s_any[4];  // of the workgroup's groups of kB pixels
+  const long long HW = (long long)a.H * a.W, total = (long long)a.B * a.C * HW;
+  if (threadIdx.x < 4) s_any[threadIdx.x] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const long long i = ((long long)block * 4 + j) * kB + threadIdx.x;
+    const int f = i < total ? a.face[i] : -1;
+    if (f < 0) continue;
+    const int view = (int)(i / HW), p = (int)(i - (long long)view * HW), y = p / a.W;
+    if (!unpack_box(a.box[(size_t)view * a.F + f]).has(p - y * a.W, y)) s_any[j] = 1;
+  }
+  __syncthreads();
+  if (threadIdx.x < 4 && s_any[threadIdx.x]) a.rest[atomicAdd(a.rest_n, 1u)] = block * 4 + threadIdx.x;
+}
+
+// dL/d(position, colour, normal) of every vertex: the records of its faces in
+// all views.  The launch's other workgroups look for what is left.
+__global__ __launch_bounds__(kB) void vertex_gather_kernel(BwdArgs a, unsigned vertex_blocks, const int* __restrict__ off,
+                                                           const int* __restrict__ lst) {
+  if (blockIdx.x >= vertex_blocks) {
+    find_rest(a, blockIdx.x - vertex_blocks);
+    return;
+  }
+  for_vertex_faces<9>(
+      off, lst, a.N, a.B,
+      [&](int b, int v, int f, float* s) {
+        const int i0 = a.faces[3 * f], i1 = a.faces[3 * f + 1], i2 = a.faces[3 * f + 2];
+        for (int c = 0; c < a.C; ++c) {
+          const size_t at = ((size_t)b * a.C + c) * a.F + f;
+          if (!(a.box[at].y >> 20)) continue;
+          const float* r = a.rec + at * a.rec_n;
+          auto corner = [&](int q) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              s[j] += r[3 * q + j];
+              if (a.rec_col) s[3 + j] += r[a.rec_col + 3 * q + j];
+              if (a.rec_vn) s[6 + j] += r[a.rec_vn + 3 * q + j];
+            }
+          };
+          if (i0 == v) corner(0);
+          if (i1 == v) corner(1);
+          if (i2 == v) corner(2);
+        }
+      },
+      [&](long long i, const float* s) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          a.g_vpos[3 * i + j] = s[j];
+          a.g_vcol[3 * i + j] = s[3 + j];
+          if (a.g_vn) a.g_vn[3 * i + j] = s[6 + j];
+        }
+      });
+}
+
+// n_v = sum over the faces around v (one entry per corner) of N_f =
+// (v1 - v0) x (v2 - v0).  With G_f = sum of dL/dn over the three corners of f,
+// dL/dv0 = (e1 - e2) x G_f, dL/dv1 = e2 x G_f, dL/dv2 = G_f x e1 (e1 = v1 - v0,
+// e2 = v2 - v0); v takes the terms of the corners it occupies.  A lane per
+// vertex took 67 us for 50k vertices (a chain of list, face and corner loads
+// for each face); eight lanes 9.
 __global__ __launch_bounds__(kB) void normal_grad_kernel(const float* __restrict__ vpos, const int* __restrict__ faces,
                                                          const int* __restrict__ off, const int* __restrict__ lst,
                                                          const float* __restrict__ g_vn, int N, int B,
                                                          float* __restrict__ g_vpos) {
+  for_vertex_faces<3>(
+      off, lst, N, B,
+      [&](int b, int v, int f, float* s) {
+        const float* vp = vpos + (size_t)b * N * 3;
+        const float* gv = g_vn + (size_t)b * N * 3;
+        const int i0 = faces[3 * f], i1 = faces[3 * f + 1], i2 = faces[3 * f + 2];
+        const f3 G = ld3(gv + 3 * i0) + ld3(gv + 3 * i1) + ld3(gv + 3 * i2);
+        const f3 p0 = ld3(vp + 3 * i0);
+        const f3 e1 = ld3(vp + 3 * i1) - p0, e2 = ld3(vp + 3 * i2) - p0;
+        f3 t = mk3(0.f, 0.f, 0.f);
+        if (i0 == v) t = t + cross(e1 - e2, G);
+        if (i1 == v) t = t + cross(e2, G);
+        if (i2 == v) t = t + cross(G, e1);
+        s[0] += t.x; s[1] += t.y; s[2] += t.z;
+      },
+      [&](long long i, const float* s) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) g_vpos[3 * i + j] += s[j];
+      });
+}
+
+// Clears two arrays and a counter.
+__global__ __launch_bounds__(kB) void clear2_kernel(float* __restrict__ p, long long n, float* __restrict__ q,
+                                                    long long m, unsigned int* counter) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)B * N) return;
-  const int b = (int)(i / N), v = (int)(i - (long long)b * N);
-  const float* vp = vpos + (size_t)b * N * 3;
-  const float* gv = g_vn + (size_t)b * N * 3;
-  f3 s = mk3(0.f, 0.f, 0.f);
-  for (int k = off[v]; k < off[v + 1]; ++k) {
-    const int fi = lst[k];
-    if (k > off[v] && lst[k - 1] == fi) continue;
-    const int i0 = faces[3 * fi], i1 = faces[3 * fi + 1], i2 = faces[3 * fi + 2];
-    const f3 G = ld3(gv + 3 * i0) + ld3(gv + 3 * i1) + ld3(gv + 3 * i2);
-    const f3 p0 = ld3(vp + 3 * i0);
-    const f3 e1 = ld3(vp + 3 * i1) - p0, e2 = ld3(vp + 3 * i2) - p0;
-    if (i0 == v) s = s + cross(e1 - e2, G);
-    if (i1 == v) s = s + cross(e2, G);
-    if (i2 == v) s = s + cross(G, e1);
-  }
-  float* o = g_vpos + 3 * i;
-  o[0] += s.x; o[1] += s.y; o[2] += s.z;
+  if (i < n) p[i] = 0.f;
+  else if (i < n + m) q[i - n] = 0.f;
+  if (counter && i == 0) *counter = 0;
+}
+
+size_t vn_floats(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B) {
+  return cfg->shading_mode == DCX_SHADING_SHADED ? 3 * (size_t)B * topo->N : 0;
+}
+int record_floats(const dcx_raster_cfg* cfg) {
+  return 9 + (cfg->albedo_mode == ALB_VERTEX_COLOR ? 9 : 0) + (cfg->shading_mode == DCX_SHADING_SHADED ? 9 : 0);
 }
 
 }  // namespace
@@ -382,7 +899,10 @@ using namespace dcx;
 
 extern "C" size_t dcx_render_bwd_workspace_size(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B) {
   if (!topo || !cfg || B <= 0) return 0;
-  return cfg->shading_mode == DCX_SHADING_SHADED ? sizeof(float) * 3 * (size_t)B * topo->N : 0;
+  const size_t faces = (size_t)B * cfg->num_cameras * topo->F;
+  const size_t pixels = (size_t)B * cfg->num_cameras * cfg->height * cfg->width;
+  return sizeof(uint2) * faces + sizeof(float) * (vn_floats(topo, cfg, B) + faces * record_floats(cfg)) +
+         sizeof(unsigned int) * ((pixels + kB - 1) / kB + 1);
 }
 
 extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B,
@@ -409,16 +929,16 @@ extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg*
               "dcx_render_bwd: textured mode needs texture + texcoords");
   DCX_REQUIRE(!(shaded || alb == ALB_TEXTURED) || vertex_normal, "dcx_render_bwd: vertex_normal required");
   DCX_REQUIRE(!shaded || sh_coeff, "dcx_render_bwd: shaded mode needs sh_coeff");
-  DCX_REQUIRE(!shaded || (workspace && workspace_bytes >= dcx_render_bwd_workspace_size(topo, cfg, B)),
-              "dcx_render_bwd: shaded mode needs a workspace of dcx_render_bwd_workspace_size() bytes");
+  const size_t vn = vn_floats(topo, cfg, B);
+  DCX_REQUIRE(!shaded || (workspace && workspace_bytes >= sizeof(float) * vn),
+              "dcx_render_bwd: shaded mode needs a workspace of at least %zu bytes", sizeof(float) * vn);
   hipStream_t s = as_stream(stream);
   const int N = topo->N, C = cfg->num_cameras;
-  DCX_HIP(hipMemsetAsync(vertex_pos_grad, 0, sizeof(float) * 3 * (size_t)B * N, s));
-  DCX_HIP(hipMemsetAsync(vertex_color_grad, 0, sizeof(float) * 3 * (size_t)B * N, s));
-  if (texture_grad && tex_h > 0 && tex_w > 0)
-    DCX_HIP(hipMemsetAsync(texture_grad, 0, sizeof(float) * 3 * (size_t)B * tex_h * tex_w, s));
-  if (sh_coeff_grad) DCX_HIP(hipMemsetAsync(sh_coeff_grad, 0, sizeof(float) * 27 * (size_t)B * C, s));
-  if (shaded) DCX_HIP(hipMemsetAsync(workspace, 0, sizeof(float) * 3 * (size_t)B * N, s));
+  // the gather form wherever its records fit the workspace
+  const bool gather = workspace && workspace_bytes >= dcx_render_bwd_workspace_size(topo, cfg, B) &&
+                      ((uintptr_t)workspace & 7) == 0 && (long long)B * C <= 65535;  // (a grid row per view)
+  const long long tex_n = texture_grad && tex_h > 0 && tex_w > 0 ? 3ll * B * tex_h * tex_w : 0;
+  const long long sh_n = sh_coeff_grad ? 27ll * B * C : 0;
   BwdArgs a{};
   a.B = B; a.C = C; a.N = N; a.F = topo->F; a.H = cfg->height; a.W = cfg->width;
   a.albedo = alb; a.shaded = shaded ? 1 : 0; a.TH = tex_h; a.TW = tex_w;
@@ -429,11 +949,44 @@ extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg*
   a.ext = extrinsics; a.intr = intrinsics;
   a.g_vpos = vertex_pos_grad; a.g_vcol = vertex_color_grad; a.g_tex = texture_grad;
   a.g_sh = shaded ? sh_coeff_grad : nullptr;
-  a.g_vn = shaded ? (float*)workspace : nullptr;
-  const long long total = (long long)B * C * cfg->height * cfg->width;
-  hipLaunchKernelGGL(render_bwd_kernel, dim3(ceil_div(total, kB)), dim3(kB), 0, s, a);
+  // workspace: [boxes] normals [records, groups left over]
+  const size_t faces = (size_t)B * C * topo->F;
+  float* ws = (float*)workspace + (gather ? 2 * faces : 0);
+  a.g_vn = shaded ? ws : nullptr;
+  const unsigned pixels = ceil_div((long long)B * C * cfg->height * cfg->width, kB);
+  auto clear = [&](float* p, long long n, float* q, long long m, unsigned int* counter) {
+    if (n + m || counter)
+      hipLaunchKernelGGL(clear2_kernel, dim3(ceil_div(n + m + 1, kB)), dim3(kB), 0, s, p, n, q, m, counter);
+  };
+  const unsigned vertices = ceil_div((long long)B * N * kVertexLanes, kB);
+  if (gather) {
+    a.box = (uint2*)workspace;
+    a.rec = ws + vn;
+    a.rec_n = record_floats(cfg);
+    a.rec_col = alb == ALB_VERTEX_COLOR ? 9 : 0;
+    a.rec_vn = shaded ? a.rec_n - 9 : 0;
+    a.rest_n = (unsigned int*)(a.rec + faces * a.rec_n);
+    a.rest = a.rest_n + 1;
+    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, a.rest_n);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(ceil_div(topo->F, kB / kFaceLanes), (unsigned)(B * C)), dim3(kB), 0, s, a);
+    };
+    const bool tex = alb == ALB_TEXTURED;
+    if (tex && shaded) launch(face_gather_kernel<true, true>);
+    else if (tex) launch(face_gather_kernel<true, false>);
+    else if (shaded) launch(face_gather_kernel<false, true>);
+    else launch(face_gather_kernel<false, false>);
+    hipLaunchKernelGGL(vertex_gather_kernel, dim3(vertices + ceil_div(pixels, 4)), dim3(kB), 0, s, a, vertices,
+                       topo->vf_off, topo->vf_list);
+    hipLaunchKernelGGL(render_bwd_kernel<true>, dim3(pixels < 1024 ? pixels : 1024), dim3(kB), 0, s, a);
+  } else {
+    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, nullptr);
+    clear(vertex_pos_grad, 3ll * B * N, vertex_color_grad, 3ll * B * N, nullptr);
+    clear(ws, (long long)vn, nullptr, 0, nullptr);
+    hipLaunchKernelGGL(render_bwd_kernel<false>, dim3(pixels), dim3(kB), 0, s, a);
+  }
   if (shaded)
-    hipLaunchKernelGGL(normal_grad_kernel, dim3(ceil_div((long long)B * N, kB)), dim3(kB), 0, s, vertex_pos,
-                       topo->faces, topo->vf_off, topo->vf_list, (const float*)workspace, N, B, vertex_pos_grad);
+    hipLaunchKernelGGL(normal_grad_kernel, dim3(vertices), dim3(kB), 0, s, vertex_pos, topo->faces, topo->vf_off,
+                       topo->vf_list, ws, N, B, vertex_pos_grad);
   return check_launch("dcx_render_bwd");
 }

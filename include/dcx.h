@@ -277,8 +277,9 @@ dcx_status dcx_render_normal_map(const dcx_topo* topo, const dcx_raster_cfg* cfg
  *   render_grad [B,C,H,W,3]; vertex_normal, barycentric, face: forward outputs
  *   outputs (overwritten): vertex_pos_grad [B,N,3], vertex_color_grad [B,N,3],
  *   texture_grad [B,TH,TW,3] (may be NULL), sh_coeff_grad [B,C,27] (may be NULL)
- *   workspace: dcx_render_bwd_workspace_size() bytes (0, so NULL allowed, when
- *   shadeless)
+ *   workspace: dcx_render_bwd_workspace_size() bytes; with less (none when
+ *   shadeless, 12 * B * N bytes when shaded) the sums are made with atomics,
+ *   which takes several times as long
  */
 size_t dcx_render_bwd_workspace_size(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B);
 dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B,

@@ -239,3 +239,61 @@ def test_binning_of_small_large_and_scattered_triangles(W, H, order):
     for got, ref in ((face, of), (bary, ob), (render, orr), (vn, ovn)):
         assert np.array_equal(got.cpu().numpy().reshape(np.shape(ref)), ref)
     assert (of >= 0).mean() > 0.3
+
+
+def _backward_with(ws_bytes, topo, cfg, g, V, col, tex, sh, tgt, vn, bary, face, ext, intr):
+    """dcx_render_bwd with a workspace of that many bytes (None: as many as it asks for)."""
+    import ctypes
+    from deepcharacters_amd import _lib
+    B, N = V.shape[:2]
+    full = _lib.load().dcx_render_bwd_workspace_size(topo.handle, ctypes.byref(cfg), B)
+    ws = torch.full((max(full if ws_bytes is None else ws_bytes, 1),), 0xff, dtype=torch.uint8, device="cuda")  # NaNs
+    out = [torch.full_like(V, float("nan")), torch.full_like(V, float("nan")),
+           None if tex is None else torch.full_like(tex, float("nan")), torch.full((B, cfg.num_cameras, 27), float("nan"), device="cuda")]
+    p = lambda x: None if x is None else x.data_ptr()
+    th, tw = (0, 0) if tex is None else tex.shape[1:3]
+    _lib.call("dcx_render_bwd", topo.handle, ctypes.byref(cfg), B, p(g), p(V), p(col), p(tex), th, tw, p(sh), p(tgt),
+              p(vn), p(bary), p(face), p(ext), p(intr), *[p(o) for o in out], p(ws) if ws_bytes != 0 else None,
+              ws.numel() if ws_bytes != 0 else 0, torch.cuda.current_stream().cuda_stream)
+    return [o for o in out if o is not None]
+
+
+@pytest.mark.parametrize("albedo,shading", [("vertexColor", "shadeless"), ("vertexColor", "shaded"),
+                                            ("textured", "shadeless"), ("textured", "shaded"), ("foregroundMask", "shadeless")])
+@pytest.mark.parametrize("buffers", ["rendered", "shifted", "random"])
+@pytest.mark.parametrize("W,H,subdiv", [(160, 120, 3), (61, 47, 4), (300, 200, 1)])
+def test_gathered_gradients_equal_the_scattered_ones(albedo, shading, buffers, W, H, subdiv):
+    """The two forms of the backward on the same buffers: faces of a pixel and
+    of thousands (left to the scatter form), and face buffers that were not
+    rendered from these positions, whose pixels lie outside their faces' boxes.
+    Sums of the same terms in another order, and the corners' image-space sums
+    transformed once: 32-bit rounding of terms up to the largest of the sums."""
+    ch, V, col, ext, intr, tex, sh = make_scene(8, W=W, H=H)
+    ch = scenes.ellipsoid_character(subdiv, scale=(0.6, 0.45, 0.35), seed=3)
+    rng = np.random.default_rng(11)
+    B, C = V.shape[0], ext.shape[1] // 12
+    V = np.stack([ch.verts + rng.normal(scale=0.005, size=ch.verts.shape) for _ in range(B)])
+    Vt, colt, extt, intrt, sht = _t(V), _t(np.stack([ch.colors] * B)), _t(ext), _t(intr), _t(sh)
+    text = _t(tex) if albedo == "textured" else None
+    topo = renderer.Topology(ch.faces, ch.N, ch.texcoords)
+    cfg = renderer.make_cfg(C, W, H, albedo, shading)
+    bary, face, render, vn = renderer.render_forward(topo, cfg, Vt, colt, text, sht, extt, intrt)
+    if buffers == "shifted":
+        face, bary = face.roll((2, 3), (2, 3)).contiguous(), bary.roll((2, 3), (2, 3)).contiguous()
+    elif buffers == "random":
+        face = torch.where(torch.rand(face.shape, device="cuda") < 0.2, torch.randint(0, ch.F, face.shape, device="cuda"), -1).int()
+        bary = torch.rand(bary.shape, device="cuda") * 0.5
+    g, tgt = _t(rng.normal(size=render.shape)), _t(rng.uniform(0, 1, render.shape))
+    args = (topo, cfg, g, Vt, colt, text, sht, tgt, vn, bary, face, extt, intrt)
+    small = 12 * B * ch.N if shading == "shaded" else 0
+    gathered, scattered = _backward_with(None, *args), _backward_with(small, *args)
+    assert int((face >= 0).sum()) > 100
+    for a, b in zip(gathered, scattered):
+        assert torch.isfinite(b).all() or buffers != "rendered"
+        ok = torch.isfinite(b)
+        assert torch.equal(ok, torch.isfinite(a))
+        assert float((a - b)[ok].abs().max()) <= 2e-4 * max(float(b[ok].abs().max()), 1e-12)
+    if albedo != "textured":  # no atomics but the SH gradients': the same bits again
+        again = _backward_with(None, *args)
+        if buffers == "rendered" and subdiv >= 3:
+            assert all(torch.equal(a, b) for a, b in zip(gathered[:2], again[:2]))
