@@ -261,11 +261,15 @@ __device__ __forceinline__ void nearest_of_wave(float& bd, int& best) {
   if (m != 0xffffffffu) bd = __uint_as_float(m);
 }
 
+// The views lie along the grid's second dimension, which ends at kMaxViewRows;
+// a launch for more of them goes on with the next kMaxViewRows in its workgroups.
+constexpr int kMaxViewRows = 65535;
+
 // The boundary pixels' indices into their view's list, one reservation per
 // workgroup; every other pixel gets its empty result.
-__global__ __launch_bounds__(kB) void sil_pixel_list_kernel(SilArgs a, GridArgs g) {
+__device__ __forceinline__ void sil_pixel_list_view(const SilArgs& a, const GridArgs& g, int view) {
   __shared__ unsigned int s_n, s_at;
-  const int view = blockIdx.y, UV = a.U * a.V, p = blockIdx.x * kB + threadIdx.x;
+  const int UV = a.U * a.V, p = blockIdx.x * kB + threadIdx.x;
   if (threadIdx.x == 0) s_n = 0;
   __syncthreads();
   unsigned int mine = 0;
@@ -280,6 +284,12 @@ __global__ __launch_bounds__(kB) void sil_pixel_list_kernel(SilArgs a, GridArgs 
   __syncthreads();
   if (found) g.list[(size_t)view * UV + s_at + mine] = (unsigned int)p;
 }
+__global__ __launch_bounds__(kB) void sil_pixel_list_kernel(SilArgs a, GridArgs g) {
+  for (int view = blockIdx.y; view < a.B * a.C; view += gridDim.y) {
+    sil_pixel_list_view(a, g, view);
+    __syncthreads();  // the counters are the next view's
+  }
+}
 
 // A wavefront per listed pixel.  (Contour pixels cluster: dealt out by the
 // workgroup that finds them, a few workgroups searched for a whole horizontal
@@ -288,8 +298,8 @@ __global__ __launch_bounds__(kB) void sil_pixel_list_kernel(SilArgs a, GridArgs 
 // pixel over cells as wide as the radius, 0.06 with the list; what is left is
 // the chain list -> cell offsets -> points of each search.
 constexpr int kSearchBlocks = 256;  // per view
-__global__ __launch_bounds__(kB) void sil_search_kernel(SilArgs a, GridArgs g) {
-  const int view = blockIdx.y, UV = a.U * a.V;
+__device__ __forceinline__ void sil_search_view(const SilArgs& a, const GridArgs& g, int view) {
+  const int UV = a.U * a.V;
   const unsigned int n = g.list_n[view * kListStride];
   for (unsigned int q = (blockIdx.x * kB + threadIdx.x) >> 6; q < n; q += kSearchBlocks * (kB / 64)) {
     const int p = __builtin_amdgcn_readfirstlane((int)g.list[(size_t)view * UV + q]);
@@ -314,6 +324,9 @@ __global__ __launch_bounds__(kB) void sil_search_kernel(SilArgs a, GridArgs g) {
     }
     if ((threadIdx.x & 63) == 0) write_d2m(a, (size_t)view * UV + p, view, best, ix, iy, sc);
   }
+}
+__global__ __launch_bounds__(kB) void sil_search_kernel(SilArgs a, GridArgs g) {
+  for (int view = blockIdx.y; view < a.B * a.C; view += gridDim.y) sil_search_view(a, g, view);
 }
 
 __global__ __launch_bounds__(kB) void sil_bwd_point_kernel(const float* __restrict__ g, const float* __restrict__ dtg,
@@ -591,12 +604,12 @@ extern "C" dcx_status dcx_mvsil_fwd(const float* points, const float* normals, c
   g.list_n = g.cnt + cells;
   const long long clear = cells + (long long)B * C * kListStride;
   hipLaunchKernelGGL(clear_u32_kernel, dim3(ceil_div(clear, kB)), dim3(kB), 0, s, g.cnt, clear);
-  hipLaunchKernelGGL(sil_pixel_list_kernel, dim3(ceil_div((long long)U * V, kB), (unsigned)(B * C)), dim3(kB), 0, s, a,
-                     g);
+  const unsigned rows = (unsigned)(B * C < kMaxViewRows ? B * C : kMaxViewRows);
+  hipLaunchKernelGGL(sil_pixel_list_kernel, dim3(ceil_div((long long)U * V, kB), rows), dim3(kB), 0, s, a, g);
   hipLaunchKernelGGL(sil_point_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, g);
   hipLaunchKernelGGL(sil_grid_scan_kernel, dim3((unsigned)(B * C)), dim3(1024), 0, s, g);
   hipLaunchKernelGGL(sil_grid_scatter_kernel, dim3(ceil_div(P, kB)), dim3(kB), 0, s, a, g);
-  hipLaunchKernelGGL(sil_search_kernel, dim3(kSearchBlocks, (unsigned)(B * C)), dim3(kB), 0, s, a, g);
+  hipLaunchKernelGGL(sil_search_kernel, dim3(kSearchBlocks, rows), dim3(kB), 0, s, a, g);
   return check_launch("dcx_mvsil_fwd(binned)");
 }
 

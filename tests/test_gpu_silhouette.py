@@ -192,3 +192,18 @@ def test_coverage_of_thin_huge_and_empty_triangles(H, W):
         proj, ocov = orc.mesh_coverage(f, V, ext, intr, H, W)
         assert np.array_equal(cov.cpu().numpy(), ocov) and ocov.any()
         assert np.array_equal(flags.cpu().numpy().astype(np.uint8), orc.boundary_flags(proj, ocov))
+
+
+def test_binned_search_of_more_views_than_grid_rows():
+    """65537 views of 3 x 2 pixels: the binned search as the scan of all points."""
+    B, C, N, U, V = 65537, 1, 5, 3, 2
+    rng = np.random.default_rng(9)
+    dt = np.full((B, C, U, V), 127, np.uint8)
+    dt[::3] = 90
+    crops = np.tile(np.array([0, 0, 2.0, 0, 0, 2.0 * U, 2.0 * V], np.float32), (B, C, 1))
+    args = [_t(rng.uniform(-3, 9, (B, C, N, 2))), _t(rng.normal(size=(B, C, N, 2))),
+            _t(rng.integers(0, 2, (B, C, N)), torch.uint8), _t(dt, torch.uint8), _t(crops)]
+    a = silhouette.multi_view_silhouette_loss_gpu(*args, "binned")
+    assert (a[3] >= 0).any()
+    for x, y in zip(a, silhouette.multi_view_silhouette_loss_gpu(*args, "brute")):
+        assert torch.equal(x, y)
