@@ -54,3 +54,16 @@ def test_cuda_renderer_wrapper_normal_map():
     tab = orc.texel_table(ch.texcoords.reshape(-1, 6), 64, 80)
     ref = orc.normal_map(tab, ch.faces, ch.verts.astype(np.float32), np.zeros_like(ch.verts, np.float32), "position")
     assert np.array_equal(nm[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("mode", ["normal", "position"])
+def test_normal_map_of_more_meshes_than_grid_rows(mode):
+    faces = np.array([[0, 1, 2], [0, 2, 3]], np.int32)
+    tc = np.array([[0, 0, 1, 0, 1, 1], [0, 0, 1, 1, 0, 1]], np.float32)
+    topo = renderer.Topology(faces, 4, tc)
+    V = torch.rand((65537, 4, 3), generator=torch.Generator().manual_seed(1)).cuda()
+    vn, nmap = renderer.render_normal_map(topo, renderer.make_cfg(1, 2, 2), mode, V, 3, 5)[3:]
+    tab = orc.texel_table(tc, 3, 5)
+    for b in (0, 1, 65534, 65535, 65536):
+        ref = orc.normal_map(tab, faces, V[b].cpu().numpy(), vn[b, 0].cpu().numpy(), mode)
+        assert np.array_equal(nmap[b].cpu().numpy(), ref)
