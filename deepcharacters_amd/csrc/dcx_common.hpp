@@ -65,6 +65,51 @@ __device__ __forceinline__ float wave_sum8(const float* v) {
   return t;
 }
 
+// s[0..n) += term(k) for k = k0, ..., k1 - 1, one after the other, for the lists
+// that the lanes of a wavefront walk (a vertex's faces).  term(k, base, out)
+// loads term k of the list whose owner passed `base`.  The terms of a short list
+// are loaded kBatch at a time by its lane; a list longer than kLongList (a
+// mesh's pole has a hundred faces and more) is loaded by the whole wavefront and
+// added up in the same order, since a lane that walks it load by load is the
+// last of its launch.  All lanes of the wavefront call it, those without a list
+// with k0 == k1.
+constexpr int kLongList = 16;
+template <int n, int kBatch, class Term>
+__device__ __forceinline__ void add_in_order(int k0, int k1, int base, float* s, Term term) {
+  if (k1 - k0 <= kLongList)
+    for (int k = k0; k < k1; k += kBatch) {
+      float t[kBatch][n];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) term(min(k + j, k1 - 1), base, t[j]);
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        if (k + j < k1) {
+#pragma unroll
+          for (int q = 0; q < n; ++q) s[q] += t[j][q];
+        }
+    }
+  for (unsigned long long many = __ballot(k1 - k0 > kLongList); many; many &= many - 1) {
+    const int src = __ffsll(many) - 1, lane = threadIdx.x & 63;
+    const int c0 = __builtin_amdgcn_readlane(k0, src), c1 = __builtin_amdgcn_readlane(k1, src);
+    const int cb = __builtin_amdgcn_readlane(base, src);
+    float t[n], u[n];
+#pragma unroll
+    for (int q = 0; q < n; ++q) t[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[q]), src));
+    for (int k = c0; k < c1; k += 64) {
+      term(min(k + lane, c1 - 1), cb, u);
+      const int m = min(64, c1 - k);
+      for (int j = 0; j < m; ++j) {
+#pragma unroll
+        for (int q = 0; q < n; ++q) t[q] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(u[q]), j));
+      }
+    }
+    if (lane == src) {
+#pragma unroll
+      for (int q = 0; q < n; ++q) s[q] = t[q];
+    }
+  }
+}
+
 // Smallest value of a group of 4, 16 or 64 lanes (all of them active), valid in
 // every lane: DPP row operations, which need no LDS crossbar round trip, and
 // for the whole wavefront the four rows' results through scalar registers.

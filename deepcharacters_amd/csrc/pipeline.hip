@@ -483,18 +483,24 @@ __global__ __launch_bounds__(kB) void vertex_fwd_kernel(Dev d, IO io, ClearList 
   if (io.vout) { io.vout[3 * (size_t)gv] = o.x; io.vout[3 * (size_t)gv + 1] = o.y; io.vout[3 * (size_t)gv + 2] = o.z; }
 }
 
+// Normalised sums of the faces' normals round each vertex (12 us for two
+// characters of 6k vertices, 76 for sixteen of 34k; 21 and 140 with the lanes of the
+// meshes' poles walking their faces one by one).
 __global__ __launch_bounds__(kB) void normals_kernel(Dev d) {
   const CharD c = d.ch[blockIdx.y];
-  const int v = blockIdx.x * kB + threadIdx.x;
-  if (v >= c.N) return;
-  const int gv = c.v0 + v;
+  const int v = blockIdx.x * kB + threadIdx.x, gv = c.v0 + v;
+  const bool in = v < c.N;
   const float* vb = d.vdef + 3 * (size_t)c.v0;
-  f3 s = mk3(0.f, 0.f, 0.f);
-  for (int k = d.vf_off[gv]; k < d.vf_off[gv + 1]; ++k) {
-    const int* fv = d.faces + 3 * ((size_t)c.f0 + d.vf_list[k]);
+  const int* faces = d.faces + 3 * (size_t)c.f0;
+  float t[3] = {0.f, 0.f, 0.f};
+  add_in_order<3, 4>(in ? d.vf_off[gv] : 0, in ? d.vf_off[gv + 1] : 0, 0, t, [&](int k, int, float* o) {
+    const int* fv = faces + 3 * (size_t)d.vf_list[k];
     const f3 a = ld3(vb + 3 * fv[0]), b1 = ld3(vb + 3 * fv[1]), b2 = ld3(vb + 3 * fv[2]);
-    s += cross(b1 - a, b2 - a);
-  }
+    const f3 n = cross(b1 - a, b2 - a);
+    o[0] = n.x; o[1] = n.y; o[2] = n.z;
+  });
+  if (!in) return;
+  const f3 s = mk3(t[0], t[1], t[2]);
   const float l = sqrtf(dot(s, s));
   const f3 n = l > 0.f ? mk3(s.x / l, s.y / l, s.z / l) : mk3(0.f, 0.f, 0.f);
   d.vnrm[3 * (size_t)gv] = n.x; d.vnrm[3 * (size_t)gv + 1] = n.y; d.vnrm[3 * (size_t)gv + 2] = n.z;
@@ -2027,21 +2033,25 @@ __global__ __launch_bounds__(kB) void vertex_bwd_kernel(Dev d, IO io) {
   if (!io.skA)
     for (int i = threadIdx.x; i < c.J * 8; i += kB) s_tab[i] = io.dq[(size_t)c.j0 * 8 + i];
   __syncthreads();
-  const int v = blockIdx.x * kB + threadIdx.x;
-  if (v >= c.N) return;
-  const int gv = c.v0 + v;
+  const int v = blockIdx.x * kB + threadIdx.x, gv = c.v0 + v;
+  const bool in = v < c.N;
   f3 g = mk3(0.f, 0.f, 0.f);
   if (!SIL) {
-    g = ld3(d.g_v + 3 * (size_t)gv);
-    f3 gc = ld3(io.g_col + 3 * (size_t)gv);
-    for (int q = d.vf_off[gv]; q < d.vf_off[gv + 1]; ++q) {
+    float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (in) {
+      const f3 g0 = ld3(d.g_v + 3 * (size_t)gv), c0 = ld3(io.g_col + 3 * (size_t)gv);
+      t[0] = g0.x; t[1] = g0.y; t[2] = g0.z; t[3] = c0.x; t[4] = c0.y; t[5] = c0.z;
+    }
+    add_in_order<6, 4>(in ? d.vf_off[gv] : 0, in ? d.vf_off[gv + 1] : 0, 0, t, [&](int q, int, float* o) {
       const float2* r = reinterpret_cast<const float2*>(d.corner_sum + 6 * (size_t)q);
       const float2 r0 = r[0], r1 = r[1], r2 = r[2];
-      g += mk3(r0.x, r0.y, r1.x);
-      gc += mk3(r1.y, r2.x, r2.y);
-    }
-    io.g_col[3 * (size_t)gv] = gc.x; io.g_col[3 * (size_t)gv + 1] = gc.y; io.g_col[3 * (size_t)gv + 2] = gc.z;
+      o[0] = r0.x; o[1] = r0.y; o[2] = r1.x; o[3] = r1.y; o[4] = r2.x; o[5] = r2.y;
+    });
+    if (!in) return;
+    g = mk3(t[0], t[1], t[2]);
+    io.g_col[3 * (size_t)gv] = t[3]; io.g_col[3 * (size_t)gv + 1] = t[4]; io.g_col[3 * (size_t)gv + 2] = t[5];
   } else {
+    if (!in) return;
     const f3 X = ld3(d.vdef + 3 * (size_t)gv);
     bool any = false;
     for (int k = 0; k < c.C; ++k) {

@@ -95,46 +95,21 @@ __global__ __launch_bounds__(kB) void face_normal_kernel(const float* __restrict
 }
 
 // Sum of face normals over each vertex's faces (increasing face order);
-// also broadcast into the [B,C,N,3] vertex_normal output when given.  A
-// vertex's loads are issued eight at a time; the few vertices with more than
-// kManyFaces faces (the poles of a mesh: a hundred and more) are loaded by the
-// whole wavefront and added up in the same order, since a lane that walks such
-// a list load by load is the last of the launch (24 us for 50k vertices and 8
-// views; with the tile counts in the same launch 24 now).  All lanes of a
-// wavefront call it.
-constexpr int kManyFaces = 16;
+// also broadcast into the [B,C,N,3] vertex_normal output when given.  One load
+// after the other, the lanes of the mesh's poles were the last of the launch
+// (24 us for 50k vertices and 8 views; with the tile counts in the same launch
+// 24 now).  All lanes of a wavefront call it.
 __device__ __forceinline__ void vertex_normal_one(const float* __restrict__ fn, const int* __restrict__ off,
                                                   const int* __restrict__ lst, int N, int F, int B, int C,
                                                   long long i, float* __restrict__ vn, float* __restrict__ vn_out) {
   const bool in = i < (long long)B * N;
   const int b = in ? (int)(i / N) : 0, v = in ? (int)(i - (long long)b * N) : 0;
-  const float* fb = fn + (size_t)b * F * 3;
-  const int k0 = in ? off[v] : 0, k1 = in ? off[v + 1] : 0;
-  f3 s = mk3(0.f, 0.f, 0.f);
-  if (k1 - k0 <= kManyFaces)
-    for (int k = k0; k < k1; k += 8) {
-      f3 n[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) n[j] = ld3(fb + 3 * lst[min(k + j, k1 - 1)]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (k + j < k1) s = s + n[j];
-    }
-  for (unsigned long long many = __ballot(k1 - k0 > kManyFaces); many; many &= many - 1) {
-    const int src = __ffsll(many) - 1, lane = threadIdx.x & 63;
-    const int c0 = __builtin_amdgcn_readlane(k0, src), c1 = __builtin_amdgcn_readlane(k1, src);
-    const float* cb = fn + (size_t)__builtin_amdgcn_readlane(b, src) * F * 3;
-    f3 t = mk3(0.f, 0.f, 0.f);
-    for (int k = c0; k < c1; k += 64) {
-      const f3 n = ld3(cb + 3 * lst[min(k + lane, c1 - 1)]);
-      const int m = min(64, c1 - k);
-      for (int j = 0; j < m; ++j)
-        t = t + mk3(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.x), j)),
-                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.y), j)),
-                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.z), j)));
-    }
-    if (lane == src) s = t;
-  }
+  float t[3] = {0.f, 0.f, 0.f};
+  add_in_order<3, 8>(in ? off[v] : 0, in ? off[v + 1] : 0, b, t, [=](int k, int mesh, float* o) {
+    const f3 n = ld3(fn + ((size_t)mesh * F + lst[k]) * 3);
+    o[0] = n.x; o[1] = n.y; o[2] = n.z;
+  });
+  const f3 s = mk3(t[0], t[1], t[2]);
   if (!in) return;
   vn[3 * i] = s.x; vn[3 * i + 1] = s.y; vn[3 * i + 2] = s.z;
   if (vn_out)

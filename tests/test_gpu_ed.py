@@ -168,3 +168,67 @@ def test_arap_truncates_neighbour_lists_at_max_connections():
     G = rng.normal(size=(1, len(nv), C, 3)).astype(np.float32)
     gT, gA = edm.embedded_graph_arap_gpu_grad(g, torch.as_tensor(G, device="cuda"), rot)
     assert torch.isfinite(gT).all() and torch.isfinite(gA).all()
+
+
+def test_normals_of_vertices_with_many_faces():
+    """Fans of 1 to 130 faces round a hub: lists at the edges of the batched and
+    of the whole-wavefront sums.  A sum of k terms in 32 bits is within
+    (k - 1) eps of the sum of their lengths; the face normals add a few eps each."""
+    degrees = [1, 3, 4, 5, 15, 16, 17, 63, 64, 65, 128, 130] * 3
+    rng = np.random.default_rng(8)
+    verts, faces = [], []
+    for k in degrees:
+        a = 2 * np.pi * np.arange(k + 1) / (k + 1)
+        hub = len(verts)
+        verts += [[0, 0, 0.4]] + [[np.cos(x), np.sin(x), rng.uniform(-0.2, 0.2)] for x in a]
+        faces += [[hub, hub + 1 + j, hub + 2 + j] for j in range(k)]
+    verts, faces = np.array(verts, np.float32), np.array(faces, np.int32)
+    N, B = len(verts), 3
+    g = scenes.EmbeddedGraph(np.zeros(1, np.int32), np.arange(N + 1, dtype=np.int32), np.zeros(N, np.int32),
+                             np.ones(N, np.float32))
+    gd = edm.GraphData(verts, g, topology=renderer.Topology(faces, N))
+    z = torch.zeros((B, 1, 3), device="cuda")
+    v, n, *_ = edm.embedded_graph_gpu(gd, z, z, z, _t(rng.uniform(-1, 1, (B, 1, 3))),
+                                      _t(rng.normal(0, 0.05, (B, N, 3))))
+    v, n = v.cpu().numpy().astype(np.float64), n.cpu().numpy()
+    for b in range(B):
+        p = v[b][faces]
+        fn = np.cross(p[:, 1] - p[:, 0], p[:, 2] - p[:, 0])
+        s, scale = np.zeros((N, 3)), np.zeros(N)
+        np.add.at(s, faces.reshape(-1), np.repeat(fn, 3, 0))
+        size = (np.linalg.norm(p[:, 1] - p[:, 0], axis=1) * np.linalg.norm(p[:, 2] - p[:, 0], axis=1))
+        np.add.at(scale, faces.reshape(-1), np.repeat(size, 3))
+        count = np.bincount(faces.reshape(-1), minlength=N)
+        length = np.linalg.norm(s, axis=1)
+        bound = np.finfo(np.float32).eps * ((count + 8) * scale / length + 4)
+        assert (np.abs(n[b] - s / length[:, None]).max(1) <= bound).all()
+
+
+@pytest.mark.parametrize("degree", [1, 15, 16, 17, 33])
+def test_arap_gradient_at_neighbour_counts_around_the_lane_group(degree):
+    M = 36
+    near = [d for h in range(1, degree // 2 + 1) for d in (h, -h)] + ([M // 2] if degree % 2 else [])
+    idx = np.array([[(i + d) % M for d in near] for i in range(M)], np.int32).reshape(-1)  # symmetric
+    off, size = np.arange(M, dtype=np.int32) * degree, np.full(M, degree, np.int32)
+    rng = np.random.default_rng(degree)
+    base = rng.normal(size=(M, 3)).astype(np.float32)
+    nv = np.arange(M, dtype=np.int32)
+    g = edm.ArapGraph(base, nv, off, size, idx, np.ones(M))
+    G = rng.normal(size=(3, M, degree, 3)).astype(np.float32)
+    dA = rng.normal(0, 0.3, (3, M, 3)).astype(np.float32)
+    for got, ref in zip(edm.embedded_graph_arap_gpu_grad(g, _t(G), _t(dA)),
+                        orc.arap_bwd(base, nv, off, size, idx, G, dA)):
+        assert _rel(got.cpu(), ref) < 1e-5
+
+
+def test_gradients_when_no_output_but_one_carries_any():
+    """Outputs without a gradient reach the backward as None."""
+    ch, g, gd, (dT, dA, sT, sA, disp), mk_node, bm, _ = setup(3)
+    args = [_t(x).requires_grad_(True) for x in (dT, dA, sT, sA, disp)]
+    edm.EmbeddedGraphGpu(gd, dT.shape[0], *args, False, "g").getNode()[2].sum().backward()  # markers alone
+    node_marker = np.full(g.num_nodes, -1, np.int32)
+    node_marker[mk_node] = np.arange(4)
+    gv, gm = np.zeros((dT.shape[0], ch.N, 3)), np.ones((dT.shape[0], 4, 3))
+    for a, ref in zip(args, orc.ed_bwd(g, ch.verts, gv, dA, sA, g_markers=gm, base_markers=bm,
+                                       node_marker=node_marker)):
+        assert float(np.abs(a.grad.cpu().numpy() - ref).max()) <= 1e-5 * max(float(np.abs(ref).max()), 1.0)
