@@ -108,6 +108,7 @@ class _EDFn(torch.autograd.Function):
         if mk is None:
             mk = torch.zeros((verts.shape[0], 0, 3), device=verts.device)
         ctx.mark_non_differentiable(nrms, graph, a_out, s_out)
+        ctx.set_materialize_grads(False)  # no zero buffers for the outputs that carry no gradient
         return verts, nrms, mk, graph, a_out, s_out
 
     @staticmethod
@@ -199,10 +200,13 @@ class ArapFn(torch.autograd.Function):
         ctx.save_for_backward(rot)
         ctx.g = g
         ctx.mark_non_differentiable(cw)
+        ctx.set_materialize_grads(False)
         return res, cw
 
     @staticmethod
     def backward(ctx, g_res, g_cw):
         (rot,) = ctx.saved_tensors
+        if g_res is None:
+            return torch.zeros_like(rot), torch.zeros_like(rot), None
         gT, gA = embedded_graph_arap_gpu_grad(ctx.g, g_res.contiguous(), rot)
         return gT, gA, None

@@ -194,12 +194,12 @@ class _RenderFn(torch.autograd.Function):
                               intrinsics, bary, face, vnorm)
         ctx.topo, ctx.cfg, ctx.albedo = topo, cfg, albedo
         ctx.mark_non_differentiable(face)
+        ctx.set_materialize_grads(False)  # no zero buffers for the outputs that carry no gradient
         return bary, face, render, vnorm
 
     @staticmethod
     def backward(ctx, g_bary, g_face, g_render, g_vnorm):
         vp, vc, tx, sh, tgt, ext, intr, bary, face, vnorm = ctx.saved_tensors
-        zeros = [None if t is None else torch.zeros_like(t) for t in (vp, vc, tx, sh)]
         if ctx.albedo in ("vertexColor", "textured") and g_render is not None:
             gvp, gvc, gtx, gsh = render_backward(ctx.topo, ctx.cfg, g_render.contiguous(), vp, vc,
                                                  tx if ctx.albedo == "textured" else None, sh, tgt, vnorm,
@@ -209,7 +209,7 @@ class _RenderFn(torch.autograd.Function):
             grads = [gvp, gvc if vc is not None else None, gtx if tx is not None else None,
                      gsh if sh is not None else None]
         else:
-            grads = zeros
+            grads = [None if t is None else torch.zeros_like(t) for t in (vp, vc, tx, sh)]
         return (*grads, None, None, None, None, None, None)
 
 

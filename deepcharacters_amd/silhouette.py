@@ -67,6 +67,7 @@ class SilhouetteFn(torch.autograd.Function):
         res, res1, dtg, cid = multi_view_silhouette_loss_gpu(points, normals, is_boundary, dt, crops, search)
         ctx.save_for_backward(dtg, cid, crops)
         ctx.mark_non_differentiable(dtg, cid)
+        ctx.set_materialize_grads(False)  # no zero buffers for the outputs that carry no gradient
         return res, res1, dtg, cid
 
     @staticmethod
