@@ -1,8 +1,8 @@
 // Rasterizer backward (CudaRendererGradGpu) on gfx950.
 //
 // Gather form (with the workspace that dcx_render_bwd_workspace_size asks for):
-// four lanes per (view, face) find the pixels of the face's box whose stored
-// face id is its own, form their contributions from the stored barycentrics
+// four lanes per (view, face), or a wavefront for the larger ones, find the
+// pixels of the face's box whose stored face id is its own, form their contributions from the stored barycentrics
 // (nothing per-pixel is kept from the forward pass besides the reference's
 // face / barycentric buffers) and sum them in registers; eight lanes per
 // vertex then add up the records of its faces in all views.  No atomics but
@@ -24,6 +24,8 @@
 // vertices' faces apply the face-normal Jacobians (RendererUtil.h:492-540) --
 // a deterministic gather in place of the reference's per-pixel loop over the
 // faces around each corner.
+#include <type_traits>
+
 #include "raster_common.hpp"
 #include "raster_internal.hpp"
 
@@ -58,14 +60,20 @@ struct BwdArgs {
   uint2* box;             // [B,C,F] a face's box: x0 | y0 << 16, nx | ny << 10 | (record written) << 20
   unsigned int* rest_n;   // pixel groups left to the scatter form, and
   unsigned int* rest;     // which ([pixels / kB] at most)
+  unsigned int* wide_n;   // [B,C], kWideStride apart: faces left to a wavefront each, and
+  unsigned int* wide;     // [B,C,F] which
   int rec_n, rec_col, rec_vn;
 };
 
 // Faces whose box holds more pixels are left to the scatter form, where a
 // large triangle's pixels are spread over many wavefronts and its long runs
-// combine well (a wavefront of the gather that held only such faces, the caps
-// of a limb, took 4 ms).
-constexpr int kGatherBox = 256;
+// combine well.  Below that, a face with a box of more than kLaneBox pixels or
+// more than kLaneHits pixels a lane takes a wavefront: large faces lie together
+// (the caps of a limb), so the wavefronts that hold them would be the last.
+constexpr int kGatherBox = 1023;  // (nx and ny are stored in 10 bits)
+constexpr int kLaneBox = 256;
+constexpr int kLaneHits = 6;
+constexpr int kWideStride = 32;   // counters that many workgroups add to, 128 bytes apart
 constexpr int kFaceLanes = 4;
 
 // Pixels that a face can cover: centres in the bounding box of its projection
@@ -438,27 +446,23 @@ __global__ __launch_bounds__(kB) void render_bwd_kernel(BwdArgs a) {
 // Sums of one face's pixels in one view.
 template <bool kTex, bool kShaded>
 struct FaceSums {
-  float gu[3], gv[3], giz[3];  // dL/d(image position, 1/z) of the corners through the barycentrics
-  f3 gx[3];                    // dL/d(world position) through the target's gradient
-  f3 gc[kTex ? 1 : 3];         // dL/d(vertex colour)
-  f3 gn[kShaded ? 3 : 1];      // dL/d(vertex normal)
-  float sh[kShaded ? 27 : 1];
+  f3 gh[3];                // dL/d(the corners' homogeneous image points K [R | t] X)
+  f3 gc[kTex ? 1 : 3];     // dL/d(vertex colour)
+  f3 gn[kShaded ? 3 : 1];  // dL/d(vertex normal)
   __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) { gu[i] = gv[i] = giz[i] = 0.f; gx[i] = mk3(0.f, 0.f, 0.f); }
+    for (int i = 0; i < 3; ++i) gh[i] = mk3(0.f, 0.f, 0.f);
 #pragma unroll
     for (int i = 0; i < (kTex ? 1 : 3); ++i) gc[i] = mk3(0.f, 0.f, 0.f);
 #pragma unroll
     for (int i = 0; i < (kShaded ? 3 : 1); ++i) gn[i] = mk3(0.f, 0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < (kShaded ? 27 : 1); ++i) sh[i] = 0.f;
   }
 };
 
 // What a face's pixels share.
 template <bool kTex, bool kShaded>
 struct FaceInfo {
-  f3 X[3], vn[kTex || kShaded ? 3 : 1], col[kTex ? 1 : 3];
+  f3 vn[kTex || kShaded ? 3 : 1], col[kTex ? 1 : 3];
   f4 p[3];
   float t6[kTex ? 6 : 1];
   FaceBox box;
@@ -469,7 +473,6 @@ struct FaceInfo {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int v = a.faces[3 * f + k];
-      X[k] = ld3(vp + 3 * v);
       p[k] = project_vertex(E, K, vp + 3 * v);
       if (kTex || kShaded) vn[k] = ld3(a.vnormal + ((size_t)view * a.N + v) * 3);
       if (!kTex) col[k] = ld3(a.vcol + ((size_t)b * a.N + v) * 3);
@@ -483,9 +486,10 @@ struct FaceInfo {
 
 // Adds pixel (x, y) of the face to its sums; the same terms as in
 // render_bwd_kernel, with what is linear in the pixels left to face_record.
+// sh: the lane's 27 sums of the SH gradient, kB floats apart.
 template <bool kTex, bool kShaded>
 __device__ __forceinline__ void add_pixel(const BwdArgs& a, int view, int b, const FaceInfo<kTex, kShaded>& I, int x,
-                                          int y, FaceSums<kTex, kShaded>& S) {
+                                          int y, FaceSums<kTex, kShaded>& S, float* sh) {
   const long long HW = (long long)a.H * a.W, i = (long long)view * HW + (long long)y * a.W + x;
   const float px = (float)x + 0.5f, py = (float)y + 0.5f;
   const float* E = a.ext + (size_t)view * 12;
@@ -548,7 +552,7 @@ __device__ __forceinline__ void add_pixel(const BwdArgs& a, int view, int b, con
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) S.sh[9 * ch + k] += gc[ch] * basis[k];
+      for (int k = 0; k < 9; ++k) sh[(9 * ch + k) * kB] += gc[ch] * basis[k];
       const float* s = shc + 9 * ch;
       const f3 Jn = mk3(s[3] + s[4] * n.y + s[7] * n.z + s[8] * 2.f * n.x,
                         s[1] + s[4] * n.x + s[5] * n.z + s[8] * -2.f * n.y,
@@ -565,7 +569,8 @@ __device__ __forceinline__ void add_pixel(const BwdArgs& a, int view, int b, con
       S.gn[k] = S.gn[k] + gun * w[k];
     }
   }
-  // through the barycentrics to the corners' image positions and 1/z (bary_vjp)
+  // through the barycentrics to the corners' image positions and 1/z
+  // (bary_vjp), and from there to their homogeneous image points
   float e[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -578,58 +583,55 @@ __device__ __forceinline__ void add_pixel(const BwdArgs& a, int view, int b, con
   const float g0 = gw[0] - gw[2], g1 = gw[1] - gw[2];
   const float s = g0 * b0 + g1 * b1;
   const float gq[3] = {(g0 - s) / Q, (g1 - s) / Q, (0.f - s) / Q};
+  float tu[3] = {0.f, 0.f, 0.f}, tv[3] = {0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int jj = k == 2 ? 0 : k + 1, kk = k == 0 ? 2 : k - 1;
     const f4 pj = I.p[jj], pk = I.p[kk];
-    S.giz[k] += gq[k] * e[k];
     const float ge = gq[k] * I.p[k].w;
-    S.gu[jj] += ge * (pk.y - py);
-    S.gv[jj] += ge * (px - pk.x);
-    S.gu[kk] += ge * (py - pj.y);
-    S.gv[kk] += ge * (pj.x - px);
+    tu[jj] += ge * (pk.y - py);
+    tv[jj] += ge * (px - pk.x);
+    tu[kk] += ge * (py - pj.y);
+    tv[kk] += ge * (pj.x - px);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const f4 p = I.p[k];
+    S.gh[k] = S.gh[k] + mk3(tu[k] * p.w, tv[k] * p.w, -((tu[k] * p.x + tv[k] * p.y) + gq[k] * e[k] * p.w) * p.w);
   }
   if (a.target) {
     f3 du, dv;
     image_gradient(a.target + (size_t)view * HW * 3, (float)x, (float)y, a.W, a.H, a.img_fs, du, dv);
     const float gu = -dot(g, du), gvv = -dot(g, dv);
-    const f3 fp = I.X[0] * w[0] + I.X[1] * w[1] + I.X[2] * w[2];
-    const float xc = E[0] * fp.x + E[1] * fp.y + E[2] * fp.z + E[3];
-    const float yc = E[4] * fp.x + E[5] * fp.y + E[6] * fp.z + E[7];
-    const float zc = E[8] * fp.x + E[9] * fp.y + E[10] * fp.z + E[11];
-    const float hx = K[0] * xc + K[1] * yc + K[2] * zc;
-    const float hy = K[3] * xc + K[4] * yc + K[5] * zc;
-    const float hz = K[6] * xc + K[7] * yc + K[8] * zc;
+    // the fragment's homogeneous image point: the projection is linear, so it
+    // is the same blend of the corners' (a gathered face's corners are all in
+    // front of the camera)
+    const float z0 = I.p[0].z * w[0], z1 = I.p[1].z * w[1], z2 = I.p[2].z * w[2];
+    const float hx = I.p[0].x * z0 + I.p[1].x * z1 + I.p[2].x * z2;
+    const float hy = I.p[0].y * z0 + I.p[1].y * z1 + I.p[2].y * z2;
+    const float hz = z0 + z1 + z2;
     if (fabsf(hz) > 0.0001f) {
-      const float gh0 = gu / hz, gh1 = gvv / hz, gh2 = -(gu * hx + gvv * hy) / (hz * hz);
-      const float cx = K[0] * gh0 + K[3] * gh1 + K[6] * gh2;
-      const float cy = K[1] * gh0 + K[4] * gh1 + K[7] * gh2;
-      const float cz = K[2] * gh0 + K[5] * gh1 + K[8] * gh2;
-      const f3 gX = mk3(E[0] * cx + E[4] * cy + E[8] * cz, E[1] * cx + E[5] * cy + E[9] * cz,
-                        E[2] * cx + E[6] * cy + E[10] * cz);
+      const f3 gf = mk3(gu / hz, gvv / hz, -(gu * hx + gvv * hy) / (hz * hz));
 #pragma unroll
-      for (int k = 0; k < 3; ++k) S.gx[k] = S.gx[k] + gX * w[k];
+      for (int k = 0; k < 3; ++k) S.gh[k] = S.gh[k] + gf * w[k];
     }
   }
 }
 
 // The face's record: its corners' image-space sums taken to world space once.
 template <bool kTex, bool kShaded>
-__device__ __forceinline__ void face_record(const BwdArgs& a, int view, const FaceInfo<kTex, kShaded>& I,
-                                            const FaceSums<kTex, kShaded>& S, float* r) {
+__device__ __forceinline__ void face_record(const BwdArgs& a, int view, const FaceSums<kTex, kShaded>& S, float* r) {
   const float* E = a.ext + (size_t)view * 12;
   const float* K = a.intr + (size_t)view * 9;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    const f4 p = I.p[i];
-    const float gh0 = S.gu[i] / p.z, gh1 = S.gv[i] / p.z;
-    const float gh2 = -(S.gu[i] * p.x + S.gv[i] * p.y) / p.z - S.giz[i] * p.w * p.w;
-    const float gx = K[0] * gh0 + K[3] * gh1 + K[6] * gh2;
-    const float gy = K[1] * gh0 + K[4] * gh1 + K[7] * gh2;
-    const float gz = K[2] * gh0 + K[5] * gh1 + K[8] * gh2;
-    r[3 * i] = E[0] * gx + E[4] * gy + E[8] * gz + S.gx[i].x;
-    r[3 * i + 1] = E[1] * gx + E[5] * gy + E[9] * gz + S.gx[i].y;
-    r[3 * i + 2] = E[2] * gx + E[6] * gy + E[10] * gz + S.gx[i].z;
+    const f3 h = S.gh[i];
+    const float gx = K[0] * h.x + K[3] * h.y + K[6] * h.z;
+    const float gy = K[1] * h.x + K[4] * h.y + K[7] * h.z;
+    const float gz = K[2] * h.x + K[5] * h.y + K[8] * h.z;
+    r[3 * i] = E[0] * gx + E[4] * gy + E[8] * gz;
+    r[3 * i + 1] = E[1] * gx + E[5] * gy + E[9] * gz;
+    r[3 * i + 2] = E[2] * gx + E[6] * gy + E[10] * gz;
     if (!kTex && a.rec_col) {
       float* c = r + a.rec_col + 3 * i;
       c[0] = S.gc[i].x; c[1] = S.gc[i].y; c[2] = S.gc[i].z;
@@ -641,100 +643,184 @@ __device__ __forceinline__ void face_record(const BwdArgs& a, int view, const Fa
   }
 }
 
-// Sums of every member but the SH gradients over a face's lanes, in all of them.
+// Sums of every member over a face's lanes, or the wavefront's, in all of them.
 template <bool kTex, bool kShaded>
-__device__ __forceinline__ void lanes_total(FaceSums<kTex, kShaded>& S) {
+__device__ __forceinline__ void lanes_total(FaceSums<kTex, kShaded>& S, bool wavefront) {
   static_assert(kFaceLanes == 4, "a quad");
-  auto sum4 = [](float v) {
+  auto sum = [=](float& v) {
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));  // 1 apart
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));  // 2 apart
-    return v;
+    if (wavefront)
+#pragma unroll
+      for (int o = 4; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
   };
-  auto f3sum = [&](f3 v) { return mk3(sum4(v.x), sum4(v.y), sum4(v.z)); };
+  auto f3sum = [&](f3& v) { sum(v.x); sum(v.y); sum(v.z); };
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    S.gu[i] = sum4(S.gu[i]); S.gv[i] = sum4(S.gv[i]); S.giz[i] = sum4(S.giz[i]);
-    S.gx[i] = f3sum(S.gx[i]);
-    if (!kTex) S.gc[i] = f3sum(S.gc[i]);
-    if (kShaded) S.gn[i] = f3sum(S.gn[i]);
+    f3sum(S.gh[i]);
+    if (!kTex) f3sum(S.gc[i]);
+    if (kShaded) f3sum(S.gn[i]);
   }
 }
 
-// kFaceLanes lanes per face, one view per workgroup row.  The box is searched
-// first (its face ids, four loads at a time, into a bit a pixel), so that the
-// wavefront runs the long part of the code as often as its lane with the most
-// pixels of its own, not as often as the largest box.
+// What one lane, four or a wavefront of them do for a face: pixel j of a lane is
+// pixel first + stride * j of the face's box.  The box is searched first (its
+// face ids, four loads at a time, into a bit a pixel), so that the wavefront
+// runs the long part of the code as often as its lane with the most pixels of
+// its own, not as often as the largest box.
+template <bool kTex, bool kShaded>
+struct FaceWalk {
+  FaceInfo<kTex, kShaded> I;
+  float inv_nx;
+  __device__ __forceinline__ void load(const BwdArgs& a, int view, int b, int f) {
+    I.load(a, view, b, f);
+    inv_nx = __builtin_amdgcn_rcpf((float)I.box.nx);
+  }
+  // k / nx for k < kGatherBox: (k + 1/2) / nx is at least 1 / (2 nx) away from a whole number
+  __device__ __forceinline__ int row_of(int k) const { return (int)(((float)k + 0.5f) * inv_nx); }
+  // the lane's pixels among the box's first n that are the face's, a bit each
+  template <int stride>
+  __device__ __forceinline__ unsigned long long search(const BwdArgs& a, int view, int f, int n, int first) const {
+    const int* ids = a.face + (size_t)view * a.H * a.W;
+    unsigned long long mine = 0;
+    for (int j0 = 0; j0 * stride + first < n; j0 += 4) {
+      int id[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = min((j0 + j) * stride + first, n - 1), y = row_of(k);
+        id[j] = ids[(size_t)(I.box.y0 + y) * a.W + I.box.x0 + k - y * I.box.nx];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        mine |= (unsigned long long)(id[j] == f && (j0 + j) * stride + first < n) << (j0 + j);
+    }
+    return mine;
+  }
+  template <int stride>
+  __device__ __forceinline__ void add(const BwdArgs& a, int view, int b, unsigned long long mine, int first,
+                                      FaceSums<kTex, kShaded>& S, float* sh) const {
+    while (mine) {
+      const int k = (__ffsll(mine) - 1) * stride + first, y = row_of(k);
+      mine &= mine - 1;
+      add_pixel<kTex, kShaded>(a, view, b, I, I.box.x0 + k - y * I.box.nx, I.box.y0 + y, S, sh);
+    }
+  }
+  __device__ __forceinline__ uint2 packed_box(bool any) const {
+    return make_uint2((unsigned)I.box.x0 | (unsigned)I.box.y0 << 16,
+                      (unsigned)I.box.nx | (unsigned)I.box.ny << 10 | (any ? 1u << 20 : 0u));
+  }
+};
+
+// The workgroup's SH gradient: its lanes' sums (27, kB floats apart), then one
+// atomic a value.
+struct ShLds { float total[32], lane[27 * kB]; };
+__device__ __forceinline__ void sh_clear(ShLds& L) {
+  if (threadIdx.x < 32) L.total[threadIdx.x] = 0.f;
+#pragma unroll
+  for (int k = 0; k < 27; ++k) L.lane[k * kB + threadIdx.x] = 0.f;
+  __syncthreads();
+}
+__device__ __forceinline__ void sh_flush(ShLds& L, const BwdArgs& a, int view, bool wave_has) {
+  if (wave_has) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = 8 * r + k < 27 ? L.lane[min(8 * r + k, 26) * kB + threadIdx.x] : 0.f;
+      const float t = wave_sum8(v);
+      if ((threadIdx.x & 63) < 8) atomicAdd(&L.total[8 * r + (threadIdx.x & 63)], t);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 27 && L.total[threadIdx.x] != 0.f)
+    atomicAdd(a.g_sh + (size_t)view * 27 + threadIdx.x, L.total[threadIdx.x]);
+}
+
+// kFaceLanes lanes per face, one view per workgroup row; the faces that this
+// would take long for go onto their view's list.
 // Pixel-parallel with segmented scans and up to 27 atomics a run, this part
 // took 570 us for 25k vertices, 4 views of 1024 x 1024, shaded vertex colours
-// (903 us textured, 50k vertices, 8 views of 1285 x 940); now 187 here, 29 in
-// the vertex gather and 97 for the pixels left over (413, 61 and 140).  What
-// bounds it is the latency of a pixel's loads at two wavefronts a SIMD: the
-// sums of a shaded face are 63 registers.
+// (903 us textured, 50k vertices, 8 views of 1285 x 940).  With every box up
+// to 256 pixels here, the lanes of the largest faces were the last of the
+// launch (183 us, and 87 for the pixels left over; textured 413 and 140); now
+// 97 here, 55 in face_wide_kernel, 31 in the vertex gather and 20 for the
+// pixels left over (289, 93, 51 and 22; with at most 3 pixels a lane the two
+// kernels take 81 + 102, with 12 118 + 53).  What bounds it is the latency of a pixel's loads at three
+// wavefronts a SIMD; the sums of a shaded face are 27 registers, and the 27
+// of the SH gradient are in LDS (with them in registers two wavefronts fit).
 template <bool kTex, bool kShaded>
-__global__ __launch_bounds__(kB) void face_gather_kernel(BwdArgs a) {
-  __shared__ float s_sh[32];
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(3))) void face_gather_kernel(BwdArgs a) {
+  __shared__ std::conditional_t<kShaded, ShLds, char> s_sh;
+  __shared__ unsigned int s_n, s_at;
   const int view = blockIdx.y, b = view / a.C, lane = threadIdx.x & 63, sub = threadIdx.x % kFaceLanes;
   const int f = (blockIdx.x * kB + threadIdx.x) / kFaceLanes;
   const bool in = f < a.F;
-  if (kShaded) {
-    if (threadIdx.x < 32) s_sh[threadIdx.x] = 0.f;
-    __syncthreads();
-  }
-  FaceInfo<kTex, kShaded> I;
-  I.load(a, view, b, in ? f : a.F - 1);
-  const int n = in ? I.box.nx * I.box.ny : 0;
-  // k / nx for k < kGatherBox: (k + 1/2) / nx is at least 1 / 512 away from a whole number
-  const float inv_nx = __builtin_amdgcn_rcpf((float)I.box.nx);
-  auto row_of = [&](int k) { return (int)(((float)k + 0.5f) * inv_nx); };
-  const int* ids = a.face + (size_t)view * a.H * a.W;
-  unsigned long long mine = 0;  // bit j: pixel sub + kFaceLanes * j
-  static_assert(kGatherBox <= 64 * kFaceLanes, "a bit a pixel");
-  for (int j0 = 0; j0 * kFaceLanes + sub < n; j0 += 4) {
-    int id[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = min((j0 + j) * kFaceLanes + sub, n - 1), y = row_of(k);
-      id[j] = ids[(size_t)(I.box.y0 + y) * a.W + I.box.x0 + k - y * I.box.nx];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      mine |= (unsigned long long)(id[j] == f && (j0 + j) * kFaceLanes + sub < n) << (j0 + j);
-  }
-  FaceSums<kTex, kShaded> S;
-  S.clear();
-  const bool found = mine != 0;
-  while (mine) {
-    const int k = (__ffsll(mine) - 1) * kFaceLanes + sub, y = row_of(k);
-    mine &= mine - 1;
-    add_pixel<kTex, kShaded>(a, view, b, I, I.box.x0 + k - y * I.box.nx, I.box.y0 + y, S);
-  }
+  if constexpr (kShaded) sh_clear(s_sh);
+  if (threadIdx.x == 0) s_n = 0;
+  FaceWalk<kTex, kShaded> w;
+  w.load(a, view, b, in ? f : a.F - 1);
+  const int n = in ? w.I.box.nx * w.I.box.ny : 0;
+  static_assert(kLaneBox <= 64 * kFaceLanes, "a bit a pixel");
+  unsigned long long mine = w.template search<kFaceLanes>(a, view, f, n > kLaneBox ? 0 : n, sub);
+  auto of_face = [&](bool c) { return (__ballot(c) >> (lane - sub) & ((1u << kFaceLanes) - 1u)) != 0; };
+  const bool wide = of_face(n > kLaneBox || __popcll(mine) > kLaneHits);
+  if (wide) mine = 0;
+  const bool any = of_face(mine != 0), wave_any = __ballot(mine != 0) != 0;
   const size_t at = (size_t)view * a.F + f;
-  const unsigned long long hits = __ballot(found);
-  if (hits) {
-    lanes_total<kTex, kShaded>(S);
-    const bool any = ((hits >> (lane - sub)) & ((1u << kFaceLanes) - 1u)) != 0;
-    if (sub == 0 && any) face_record<kTex, kShaded>(a, view, I, S, a.rec + at * a.rec_n);
-    if (sub == 0 && in)
-      a.box[at] = make_uint2((unsigned)I.box.x0 | (unsigned)I.box.y0 << 16,
-                             (unsigned)I.box.nx | (unsigned)I.box.ny << 10 | (any ? 1u << 20 : 0u));
-  } else if (sub == 0 && in) {
-    a.box[at] = make_uint2((unsigned)I.box.x0 | (unsigned)I.box.y0 << 16, (unsigned)I.box.nx | (unsigned)I.box.ny << 10);
+  if (wave_any) {
+    FaceSums<kTex, kShaded> S;
+    S.clear();
+    float* sh = nullptr;
+    if constexpr (kShaded) sh = s_sh.lane + threadIdx.x;
+    w.template add<kFaceLanes>(a, view, b, mine, sub, S, sh);
+    lanes_total<kTex, kShaded>(S, false);
+    if (sub == 0 && any) face_record<kTex, kShaded>(a, view, S, a.rec + at * a.rec_n);
   }
-  if (kShaded && a.g_sh) {
-    if (hits) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = 8 * r + k < 27 ? S.sh[8 * r + k < 27 ? 8 * r + k : 0] : 0.f;
-        const float t = wave_sum8(v);
-        if (lane < 8) atomicAdd(&s_sh[8 * r + lane], t);
-      }
+  if (sub == 0 && in) a.box[at] = w.packed_box(any);
+  __syncthreads();
+  unsigned int slot = 0;
+  if (sub == 0 && wide) slot = atomicAdd(&s_n, 1u);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_n) s_at = atomicAdd(a.wide_n + view * kWideStride, s_n);
+  __syncthreads();
+  if (sub == 0 && wide) a.wide[(size_t)view * a.F + s_at + slot] = (unsigned int)f;
+  if constexpr (kShaded)
+    if (a.g_sh) sh_flush(s_sh, a, view, wave_any);
+}
+
+// A wavefront per listed face of the view (a workgroup row).  (In the gather's
+// own wavefronts, one large face after the other, this took 300 us: they lie
+// together.)
+template <bool kTex, bool kShaded>
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(kTex ? 3 : 2))) void face_wide_kernel(BwdArgs a) {
+  __shared__ std::conditional_t<kShaded, ShLds, char> s_sh;
+  static_assert(kGatherBox <= 64 * 64, "a bit a pixel");
+  const int view = blockIdx.y, b = view / a.C, lane = threadIdx.x & 63;
+  const unsigned int n = a.wide_n[view * kWideStride];
+  if ((blockIdx.x * kB) >> 6 >= n) return;
+  if constexpr (kShaded) sh_clear(s_sh);
+  bool wave_any = false;
+  for (unsigned int q = (blockIdx.x * kB + threadIdx.x) >> 6; q < n; q += gridDim.x * (kB / 64)) {
+    const int f = __builtin_amdgcn_readfirstlane((int)a.wide[(size_t)view * a.F + q]);
+    FaceWalk<kTex, kShaded> w;
+    w.load(a, view, b, f);
+    const unsigned long long mine = w.template search<64>(a, view, f, w.I.box.nx * w.I.box.ny, lane);
+    if (!__ballot(mine != 0)) continue;  // its box says that there is no record
+    wave_any = true;
+    FaceSums<kTex, kShaded> S;
+    S.clear();
+    float* sh = nullptr;
+    if constexpr (kShaded) sh = s_sh.lane + threadIdx.x;
+    w.template add<64>(a, view, b, mine, lane, S, sh);
+    lanes_total<kTex, kShaded>(S, true);
+    const size_t at = (size_t)view * a.F + f;
+    if (lane == 0) {
+      face_record<kTex, kShaded>(a, view, S, a.rec + at * a.rec_n);
+      a.box[at] = w.packed_box(true);
     }
-    __syncthreads();
-    if (threadIdx.x < 27 && s_sh[threadIdx.x] != 0.f)
-      atomicAdd(a.g_sh + (size_t)view * 27 + threadIdx.x, s_sh[threadIdx.x]);
   }
+  if constexpr (kShaded)
+    if (a.g_sh) sh_flush(s_sh, a, view, wave_any);
 }
 
 constexpr int kVertexLanes = 8;
@@ -876,13 +962,14 @@ __global__ __launch_bounds__(kB) void normal_grad_kernel(const float* __restrict
       });
 }
 
-// Clears two arrays and a counter.
+// Clears two arrays and some counters.
 __global__ __launch_bounds__(kB) void clear2_kernel(float* __restrict__ p, long long n, float* __restrict__ q,
-                                                    long long m, unsigned int* counter) {
+                                                    long long m, unsigned int* __restrict__ counters,
+                                                    long long c) {
   const long long i = (long long)blockIdx.x * kB + threadIdx.x;
   if (i < n) p[i] = 0.f;
   else if (i < n + m) q[i - n] = 0.f;
-  if (counter && i == 0) *counter = 0;
+  else if (i < n + m + c) counters[i - n - m] = 0u;
 }
 
 size_t vn_floats(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B) {
@@ -902,7 +989,7 @@ extern "C" size_t dcx_render_bwd_workspace_size(const dcx_topo* topo, const dcx_
   const size_t faces = (size_t)B * cfg->num_cameras * topo->F;
   const size_t pixels = (size_t)B * cfg->num_cameras * cfg->height * cfg->width;
   return sizeof(uint2) * faces + sizeof(float) * (vn_floats(topo, cfg, B) + faces * record_floats(cfg)) +
-         sizeof(unsigned int) * ((pixels + kB - 1) / kB + 1);
+         sizeof(unsigned int) * ((pixels + kB - 1) / kB + 1 + kWideStride * (size_t)B * cfg->num_cameras + faces);
 }
 
 extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B,
@@ -954,9 +1041,9 @@ extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg*
   float* ws = (float*)workspace + (gather ? 2 * faces : 0);
   a.g_vn = shaded ? ws : nullptr;
   const unsigned pixels = ceil_div((long long)B * C * cfg->height * cfg->width, kB);
-  auto clear = [&](float* p, long long n, float* q, long long m, unsigned int* counter) {
-    if (n + m || counter)
-      hipLaunchKernelGGL(clear2_kernel, dim3(ceil_div(n + m + 1, kB)), dim3(kB), 0, s, p, n, q, m, counter);
+  auto clear = [&](float* p, long long n, float* q, long long m, unsigned int* counters, long long c) {
+    if (n + m + c)
+      hipLaunchKernelGGL(clear2_kernel, dim3(ceil_div(n + m + c, kB)), dim3(kB), 0, s, p, n, q, m, counters, c);
   };
   const unsigned vertices = ceil_div((long long)B * N * kVertexLanes, kB);
   if (gather) {
@@ -966,23 +1053,29 @@ extern "C" dcx_status dcx_render_bwd(const dcx_topo* topo, const dcx_raster_cfg*
     a.rec_col = alb == ALB_VERTEX_COLOR ? 9 : 0;
     a.rec_vn = shaded ? a.rec_n - 9 : 0;
     a.rest_n = (unsigned int*)(a.rec + faces * a.rec_n);
-    a.rest = a.rest_n + 1;
-    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, a.rest_n);
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(ceil_div(topo->F, kB / kFaceLanes), (unsigned)(B * C)), dim3(kB), 0, s, a);
+    a.wide_n = a.rest_n + 1;
+    a.wide = a.wide_n + kWideStride * (size_t)B * C;
+    a.rest = a.wide + faces;
+    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, a.rest_n, 1 + kWideStride * (long long)B * C);
+    const unsigned views = (unsigned)(B * C);
+    // as many workgroups as can be resident, and at least a few for each view's list
+    const unsigned wide = views < 192 ? 768 / views : 4;
+    auto launch = [&](auto kernel, auto wide_kernel) {
+      hipLaunchKernelGGL(kernel, dim3(ceil_div(topo->F, kB / kFaceLanes), views), dim3(kB), 0, s, a);
+      hipLaunchKernelGGL(wide_kernel, dim3(wide, views), dim3(kB), 0, s, a);
     };
     const bool tex = alb == ALB_TEXTURED;
-    if (tex && shaded) launch(face_gather_kernel<true, true>);
-    else if (tex) launch(face_gather_kernel<true, false>);
-    else if (shaded) launch(face_gather_kernel<false, true>);
-    else launch(face_gather_kernel<false, false>);
+    if (tex && shaded) launch(face_gather_kernel<true, true>, face_wide_kernel<true, true>);
+    else if (tex) launch(face_gather_kernel<true, false>, face_wide_kernel<true, false>);
+    else if (shaded) launch(face_gather_kernel<false, true>, face_wide_kernel<false, true>);
+    else launch(face_gather_kernel<false, false>, face_wide_kernel<false, false>);
     hipLaunchKernelGGL(vertex_gather_kernel, dim3(vertices + ceil_div(pixels, 4)), dim3(kB), 0, s, a, vertices,
                        topo->vf_off, topo->vf_list);
     hipLaunchKernelGGL(render_bwd_kernel<true>, dim3(pixels < 1024 ? pixels : 1024), dim3(kB), 0, s, a);
   } else {
-    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, nullptr);
-    clear(vertex_pos_grad, 3ll * B * N, vertex_color_grad, 3ll * B * N, nullptr);
-    clear(ws, (long long)vn, nullptr, 0, nullptr);
+    clear(texture_grad, tex_n, sh_coeff_grad, sh_n, nullptr, 0);
+    clear(vertex_pos_grad, 3ll * B * N, vertex_color_grad, 3ll * B * N, nullptr, 0);
+    clear(ws, (long long)vn, nullptr, 0, nullptr, 0);
     hipLaunchKernelGGL(render_bwd_kernel<false>, dim3(pixels), dim3(kB), 0, s, a);
   }
   if (shaded)

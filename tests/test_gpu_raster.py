@@ -297,3 +297,48 @@ def test_gathered_gradients_equal_the_scattered_ones(albedo, shading, buffers, W
         again = _backward_with(None, *args)
         if buffers == "rendered" and subdiv >= 3:
             assert all(torch.equal(a, b) for a, b in zip(gathered[:2], again[:2]))
+
+
+@pytest.mark.parametrize("albedo,shading", [("vertexColor", "shaded"), ("textured", "shaded"), ("textured", "shadeless"),
+                                            ("foregroundMask", "shadeless")])
+def test_gathered_gradients_at_the_edges_of_the_face_sizes(albedo, shading):
+    """Triangles whose boxes and pixel counts lie around the limits between a
+    face's own lanes, a wavefront and the scatter form: boxes of up to 16 x 16,
+    31 x 33 and 32 x 32 pixels, single rows and columns of up to 1024, a few
+    pixels (24, 28) and a single one, several views' lists of different lengths.
+    32-bit sums of the same terms, as above."""
+    W, H = 1100, 1090
+    sizes = [(1, 1), (2, 2), (7, 7), (7, 8), (8, 8), (15, 17), (16, 16), (16, 17), (17, 17), (31, 33), (32, 32), (33, 33),
+             (64, 4), (64, 5), (256, 1), (257, 1), (1, 257), (1022, 1), (1023, 1), (1024, 1), (1, 1023), (1, 1024), (40, 60)]
+    rng = np.random.default_rng(12)
+    tris, x, y, row = [], 4, 4, 0
+    for w, h in [s for s in sizes for _ in range(6)]:
+        if x + w + 2 > W - 6:
+            x, y, row = 4, y + row + 2, 0
+        if y + h + 2 < H - 6:
+            # corners on the box's outer pixels' centres, off by under half a pixel
+            c = np.array([[x, y], [x + w - 1, y + (h - 1) * rng.integers(0, 2)], [x + (w - 1) // 2, y + h - 1]])
+            tris.append(c + 0.5 + rng.uniform(-0.45, 0.45, (3, 2)))
+            x, row = x + w + 2, max(row, h)
+    xy = np.concatenate(tris)
+    z = rng.uniform(1, 1.5, len(xy))
+    V = np.concatenate([xy * z[:, None], z[:, None]], 1)[None].astype(np.float32)
+    faces = np.arange(len(xy), dtype=np.int32).reshape(-1, 3)
+    intr = np.tile(np.array([1, 0, 0, 0, 1, 0, 0, 0, 1], np.float32), 3)[None]  # (x z, y z, z) is seen at (x, y)
+    ext = np.array([[1, 0, 0, t, 0, 1, 0, 0, 0, 0, 1, 0] for t in (0, 700, -700)], np.float32).reshape(1, 36)
+    topo = renderer.Topology(faces, len(xy), rng.uniform(0.1, 0.9, (len(faces), 6)).astype(np.float32))
+    cfg = renderer.make_cfg(3, W, H, albedo, shading)
+    Vt, colt, extt, intrt = _t(V), _t(rng.uniform(0, 1, V.shape)), _t(ext), _t(intr)
+    text = _t(rng.uniform(0, 1, (1, 64, 64, 3))) if albedo == "textured" else None
+    sht = _t(rng.uniform(0.1, 0.5, (1, 3, 27)))
+    bary, face, render, vn = renderer.render_forward(topo, cfg, Vt, colt, text, sht, extt, intrt)
+    g, tgt = _t(rng.normal(size=render.shape)), _t(rng.uniform(0, 1, render.shape))
+    args = (topo, cfg, g, Vt, colt, text, sht, tgt, vn, bary, face, extt, intrt)
+    seen = torch.bincount(face[0, 0].flatten()[face[0, 0].flatten() >= 0].long(), minlength=len(faces))
+    assert int((seen > 0).sum()) > len(faces) // 2 and int(seen.max()) > 500 and int((seen == 1).sum()) > 0
+    small = 12 * V.shape[1] if shading == "shaded" else 0
+    gathered, scattered = _backward_with(None, *args), _backward_with(small, *args)
+    assert bool(scattered[0].any())
+    for a, b in zip(gathered, scattered):
+        assert torch.isfinite(b).all()
+        assert float((a - b).abs().max()) <= 2e-4 * max(float(b.abs().max()), 1e-12)
