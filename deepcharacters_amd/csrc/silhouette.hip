@@ -470,46 +470,51 @@ struct EdgeQuotient {
   }
 };
 
-// Eight lanes per (view, face), one row of its pixel box each.  A weight is
+// Four lanes per (view, face), one row of its pixel box each.  A weight is
 // compared with the limits as a product with the reciprocal, within 1e-6 of
 // the quotient where it is near them, so the two divisions are made only for
 // pixels within 1e-5 of a limit, and for triangles near the ends of the
 // exponent range.  A lane per face walked boxes of 34 x 34 pixels (the long
 // triangles of a cap, 64 of them in one wavefront) after the rest of the
-// launch was done.  16 views of 1285 x 940, 100k faces: 294 -> 107 us, which is
-// the issue time of its vector instructions.
-constexpr int kCovLanes = 8;
+// launch was done.  16 views of 1285 x 940, 100k faces: 294 -> 97 us (108 with
+// eight lanes), which is the issue time of its vector instructions.
+constexpr int kCovLanes = 4;
+constexpr unsigned kMaxCovBlocks = 1u << 23;  // more faces: several a group of lanes
 __global__ __launch_bounds__(kB) void cov_raster_kernel(const float* __restrict__ uv, const int* __restrict__ faces,
                                                          int B, int C, int N, int F, int H, int W,
                                                          unsigned char* __restrict__ cov) {
-  const long long i = ((long long)blockIdx.x * kB + threadIdx.x) / kCovLanes;
-  if (i >= (long long)B * C * F) return;
-  const int view = (int)(i / F), f = (int)(i - (long long)view * F);
-  const f2* P = (const f2*)uv + (size_t)view * N;
-  const f2 p0 = P[faces[3 * f]], p1 = P[faces[3 * f + 1]], p2 = P[faces[3 * f + 2]];
-  const float bx0 = fmaxf(fminf(p0.x, fminf(p1.x, p2.x)) - 0.5f, 0.f);
-  const float by0 = fmaxf(fminf(p0.y, fminf(p1.y, p2.y)) - 0.5f, 0.f);
-  const float bx1 = fminf(fmaxf(p0.x, fmaxf(p1.x, p2.x)) + 0.5f, (float)(W - 1));
-  const float by1 = fminf(fmaxf(p0.y, fmaxf(p1.y, p2.y)) + 0.5f, (float)(H - 1));
-  // first weights 1 at p1 and p2; e0 = 1 - e2 - e1
-  const EdgeQuotient q1(p0, p2, p1), q2(p0, p1, p2);
-  const bool plain = q1.plain() && q2.plain();
-  constexpr float kLo = -0.001f, kHi = 1.001f, kMargin = 1e-5f;
-  const int ue = bx1 >= 0.f ? (int)bx1 : -1, ve = by1 >= 0.f ? (int)by1 : -1;  // the last u, v with (float)u <= bx1
-  for (int v = (int)by0 + (int)(threadIdx.x % kCovLanes); v <= ve; v += kCovLanes) {
-    unsigned char* row = cov + (size_t)view * H * W + (size_t)v * W;
-    const float py = (float)v + 0.5f, r1 = q1.dx * py, r2 = q2.dx * py;
-    for (int u = (int)bx0; u <= ue; ++u) {
-      const float n1 = q1.num((float)u + 0.5f, r1), n2 = q2.num((float)u + 0.5f, r2);
-      const float a1 = n1 * q1.r, a2 = n2 * q2.r, a0 = 1.f - a2 - a1;
-      const float lo = fminf(a0, fminf(a1, a2)), hi = fmaxf(a0, fmaxf(a1, a2));
-      if (plain && (lo < kLo - kMargin || hi > kHi + kMargin)) continue;
-      bool in = true;
-      if (!(plain && lo > kLo + kMargin && hi < kHi - kMargin)) {
-        const float e2 = n2 / q2.den, e1 = n1 / q1.den, e0 = 1.f - e2 - e1;
-        in = e0 >= kLo && e1 >= kLo && e2 >= kLo && e0 <= kHi && e1 <= kHi && e2 <= kHi;
+  const long long n = (long long)B * C * F;
+  for (long long i = ((long long)blockIdx.x * kB + threadIdx.x) / kCovLanes; i < n;
+       i += (long long)gridDim.x * (kB / kCovLanes)) {
+    // (32-bit where it can be: a 64-bit division is some 100 instructions)
+    const int view = n < 1ll << 32 ? (int)((unsigned)i / (unsigned)F) : (int)(i / F);
+    const int f = (int)(i - (long long)view * F);
+    const f2* P = (const f2*)uv + (size_t)view * N;
+    const f2 p0 = P[faces[3 * f]], p1 = P[faces[3 * f + 1]], p2 = P[faces[3 * f + 2]];
+    const float bx0 = fmaxf(fminf(p0.x, fminf(p1.x, p2.x)) - 0.5f, 0.f);
+    const float by0 = fmaxf(fminf(p0.y, fminf(p1.y, p2.y)) - 0.5f, 0.f);
+    const float bx1 = fminf(fmaxf(p0.x, fmaxf(p1.x, p2.x)) + 0.5f, (float)(W - 1));
+    const float by1 = fminf(fmaxf(p0.y, fmaxf(p1.y, p2.y)) + 0.5f, (float)(H - 1));
+    // first weights 1 at p1 and p2; e0 = 1 - e2 - e1
+    const EdgeQuotient q1(p0, p2, p1), q2(p0, p1, p2);
+    const bool plain = q1.plain() && q2.plain();
+    constexpr float kLo = -0.001f, kHi = 1.001f, kMargin = 1e-5f;
+    const int ue = bx1 >= 0.f ? (int)bx1 : -1, ve = by1 >= 0.f ? (int)by1 : -1;  // the last u, v with (float)u <= bx1
+    for (int v = (int)by0 + (int)(threadIdx.x % kCovLanes); v <= ve; v += kCovLanes) {
+      unsigned char* row = cov + (size_t)view * H * W + (size_t)v * W;
+      const float py = (float)v + 0.5f, r1 = q1.dx * py, r2 = q2.dx * py;
+      for (int u = (int)bx0; u <= ue; ++u) {
+        const float n1 = q1.num((float)u + 0.5f, r1), n2 = q2.num((float)u + 0.5f, r2);
+        const float a1 = n1 * q1.r, a2 = n2 * q2.r, a0 = 1.f - a2 - a1;
+        const float lo = fminf(a0, fminf(a1, a2)), hi = fmaxf(a0, fmaxf(a1, a2));
+        if (plain && (lo < kLo - kMargin || hi > kHi + kMargin)) continue;
+        bool in = true;
+        if (!(plain && lo > kLo + kMargin && hi < kHi - kMargin)) {
+          const float e2 = n2 / q2.den, e1 = n1 / q1.den, e0 = 1.f - e2 - e1;
+          in = e0 >= kLo && e1 >= kLo && e2 >= kLo && e0 <= kHi && e1 <= kHi && e2 <= kHi;
+        }
+        if (in) row[u] = 1;
       }
-      if (in) row[u] = 1;
     }
   }
 }
@@ -666,11 +671,12 @@ extern "C" dcx_status dcx_projected_mesh_boundary(const dcx_topo* topo, int B, i
   float* uv = (float*)workspace;
   unsigned char* cov = coverage ? coverage : (unsigned char*)workspace + align256(sizeof(float) * 2 * (size_t)B * C * N);
   const long long npix = (long long)B * C * H * W;
+  const unsigned cov_blocks = ceil_div((long long)B * C * F, kB / kCovLanes);
   hipLaunchKernelGGL(fill_u8_kernel, dim3(ceil_div(npix, 16 * kB)), dim3(kB), 0, s, cov, npix);
   hipLaunchKernelGGL(cov_project_kernel, dim3(ceil_div((long long)B * C * N, kB)), dim3(kB), 0, s, points, extrinsics,
                      intrinsics, B, C, N, uv);
-  hipLaunchKernelGGL(cov_raster_kernel, dim3(ceil_div((long long)B * C * F, kB / kCovLanes)), dim3(kB), 0, s, uv, topo->faces, B,
-                     C, N, F, H, W, cov);
+  hipLaunchKernelGGL(cov_raster_kernel, dim3(cov_blocks < kMaxCovBlocks ? cov_blocks : kMaxCovBlocks), dim3(kB), 0, s, uv,
+                     topo->faces, B, C, N, F, H, W, cov);
   hipLaunchKernelGGL(cov_boundary_kernel, dim3(ceil_div((long long)B * C * N, kB)), dim3(kB), 0, s, cov, uv, B, C, N,
                      H, W, is_boundary);
   return check_launch("dcx_projected_mesh_boundary");
