@@ -221,7 +221,7 @@ dcx_status dcx_render_fwd(const dcx_topo* topo, const dcx_raster_cfg* cfg, int B
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): dcx_render_fwd with its scratch (projections, normals,
- * triangle records, tile counters and lists) in a static device array of
+ * tile ranges, tile counters and lists) in a static device array of
  * DCX_RENDER_NOALLOC_SCRATCH_BYTES per device instead of a caller workspace.
  * It calls no hipMalloc, hipFree or allocating library routine; its counters
  * are cleared by kernels, not memsets.  A batch whose scratch would exceed the
@@ -375,7 +375,7 @@ dcx_status dcx_arap_bwd(const float* base_pos, const int32_t* node_vertex, const
 
 /* data->model nearest boundary-point search */
 #define DCX_SIL_BRUTE 0  /* every point, as the reference */
-#define DCX_SIL_BINNED 1 /* uniform grid of 30*scale cells, identical results */
+#define DCX_SIL_BINNED 1 /* uniform grid, eight cells per search radius of 30*scale; identical results */
 
 /* Workspace bytes for dcx_mvsil_fwd with DCX_SIL_BINNED (0 on bad sizes). */
 size_t dcx_mvsil_workspace_size(int B, int C, int N, int U, int V);
